@@ -183,6 +183,14 @@ bool use_skinny(const qmoe_gemm_desc* d) {
   // dense e2m1 (MXFP4 / NVFP4): the tiled kernel's 32-token tiles with a K
   // split win from 33 rows (measured on MI355X, K 2880, N 5760)
   if (!d->group_offs && (d->kind == QMOE_W4A16_MX || d->kind == QMOE_W4A16_NV)) lim = kSkinnyMaxRowsW8A8;
+  // grouped e2m1: the tiles from as many routes as experts on (measured on
+  // MI355X, GPT-OSS MoE, 128 experts, top 4: MXFP4 16 tokens 201 us both ways,
+  // 32 / 64 / 128 / 256 tokens 346 / 447 / 514 / 590 -> 316 / 373 / 403 / 419
+  // us, NVFP4 32 / 128 tokens 399 / 612 -> 392 / 541; INT4 loses, 355 / 577 ->
+  // 407 / 597)
+  if (d->group_offs && (d->kind == QMOE_W4A16_MX || d->kind == QMOE_W4A16_NV) && d->M >= d->slots &&
+      (d->K % 64) == 0)
+    lim = 0;
   if (env) lim = atoi(env);
   return skinny_rows(d) <= lim;
 }

@@ -10,29 +10,41 @@
 // as dequantizing the whole matrix first: exact for e8m0 scales, one
 // round-to-nearest-even of value * scale for the bf16 NVFP4 / INT4 scales.
 //
-// Design for gfx950 (one workgroup of 4 wavefronts per CU), on the machinery
-// of the 1-byte tiled kernel (gemm_tile.h):
+// Design for gfx950 (w4_gemm_kernel):
 //  * output tile BM tokens x 256 weight rows of 32 x 32 MFMA blocks (weight
-//    block first, activation block second: v_mfma_f32_32x32x16_bf16);
-//  * a stage is 64 k: 128 bytes of each activation row and 32 bytes of each
-//    weight row, copied straight into a ring of four LDS stages (distinct
-//    arrays) four stages ahead; each lane loads the scale bytes it needs
-//    with the copies (bounded buffer loads into a 4-deep register ring);
+//    block first, activation block second: v_mfma_f32_32x32x16_bf16). Each of
+//    4 wavefronts owns 64 weight rows for all BM tokens, so it expands its
+//    rows once; two workgroups share a CU (80 KB of LDS, 256 VGPRs), or
+//    two K groups of 4 wavefronts share a workgroup (KG 2) where the tiles
+//    only fill one workgroup per CU: one wavefront's instructions issue in
+//    order, and it takes a second one to put the expansion of one beside the
+//    MFMAs of the other;
+//  * what bounds it: from ~1000 tokens the matrix cores and the copies into
+//    LDS beside them (K 2880, N 5760, 8192 tokens: 258 us, 1.05 PFLOP/s; MFMAs
+//    and LDS reads alone 172 us); a routed expert's few rows, the weight
+//    stream (GPT-OSS MoE, 512 / 2048 tokens 794 / 1162 -> 457 / 700 us);
+//  * a wavefront's codes are copied as whole 128-byte lines of its own rows
+//    (256 k, four stages) into its own LDS rows and from there into
+//    registers at the start of the line, which frees the buffer for the next
+//    line: 64 KB per CU stay in flight. 64-byte pieces of rows of 1440 bytes
+//    fetched 2.3 times the bytes (L2 misses 5.3 GB where the codes are 1.06
+//    GB) and were the limit. A wavefront owns every fourth row of the tile,
+//    whose lines start at the same place (see `ph`);
+//  * activations: stages of 64 k (128 bytes of each row) in a ring of three
+//    sets, copied two sets ahead, one barrier per set;
 //  * in a stage, lane l (row l % 32, half h = l / 32) feeds k in
 //    [32h, 32h + 32): that is one e8m0 block (two NVFP4 blocks), 16
-//    contiguous code bytes (one LDS read for all four 16-k MFMA steps) and
-//    one scale byte (NVFP4: one 4-byte bf16 pair; INT4: one bf16 group
-//    scale). Each 16-k step expands 8 codes to bf16 with the scale applied
-//    (v_cvt_scalef32_pk_bf16_fp4 for e8m0; unscaled conversion, f32 product
-//    and bf16 rounding for NVFP4 and INT4);
+//    contiguous code bytes and one scale byte (NVFP4: one 4-byte bf16 pair;
+//    INT4: one bf16 group scale). Each 16-k step expands 8 codes to bf16 with
+//    the scale applied (v_cvt_scalef32_pk_bf16_fp4 for e8m0; unscaled
+//    conversion, f32 product and bf16 rounding for NVFP4 and INT4);
 //    activation and weight use the same lane -> k assignment, so the
 //    products pair up whatever order the MFMA sums;
-//  * every operand of stage s+1 is read into the second register set during
-//    the MFMAs of stage s; the activation rows are stored with the 16-byte
-//    chunk c of row r at slot c ^ ((r & 7) ^ ((r >> 3) & 1)) so that the
-//    MFMA operand reads are conflict-free;
-//  * the shared epilogue applies bias, fused activation and routing weight
-//    (the weights carry no other scale).
+//  * LDS rows of 128 bytes hold the 16-byte chunk c of row r at slot
+//    c ^ ((r & 7) ^ ((r >> 3) & 1)), so that the operand reads are
+//    conflict-free;
+//  * the epilogue applies bias, fused activation and routing weight (the
+//    weights carry no other scale).
 
 #include <algorithm>
 #include <cstdlib>
@@ -43,19 +55,6 @@ namespace {
 
 using rsrc_t = __amdgpu_buffer_rsrc_t;
 constexpr int kW4BN = 256;  // weight rows per tile
-
-// The wavefronts split the 256 weight rows (each expands its own 64 rows
-// once per stage and reuses them for all BM tokens); WN = 4 always.
-template <int BM>
-struct W4Shape {
-  static constexpr int WN = 4;                  // wavefronts along weight rows
-  static constexpr int WM = 1;                  // along tokens
-  static constexpr int TN = kW4BN / WN;         // weight rows per wavefront
-  static constexpr int TM = BM / WM;            // tokens per wavefront
-  static constexpr int NI = TN / 32;
-  static constexpr int MJ = TM / 32;
-  static_assert(NI >= 1 && MJ >= 1, "tile too small");
-};
 
 __device__ __forceinline__ int w4_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
@@ -81,9 +80,468 @@ __device__ __forceinline__ bf16x8 as_bf16x8_u4(const uint4& x) {
   return c.v;
 }
 
+// One direct global -> LDS copy of 16 bytes per lane: `lds` (byte address,
+// wave-uniform) + 16 * lane <- src. Written as assembly so that the compiler
+// does not order it against the LDS reads: it would drain every copy in
+// flight before a read of a ring buffer whose index it cannot resolve. The
+// kernel's own counted waits and barriers order them. The instruction has no
+// register result and takes its address registers when it issues; the
+// s_nop is the wait state between a write of M0 and its use.
+__device__ __forceinline__ void w4_copy16(const uint8_t* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
+}
+__device__ __forceinline__ void w4_copy16(const uint8_t* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
+               : "memory", "m0");
+}
+
 // FMT: 0 MXFP4, 1 NVFP4, 2 INT4
+template <int BM, int KG, bool ACT, int FMT>
+__global__ __launch_bounds__(KG * kThreads, 2) void w4_gemm_kernel(const GemmParams p, int m_tiles, int n_tiles) {
+  constexpr bool NV = FMT == 1, I4 = FMT == 2;
+  constexpr int BN = kW4BN;
+  constexpr int NI = 2, MJ = BM / 32;     // 32-row weight blocks, 32-token blocks per wavefront
+  constexpr int BNO = ACT ? BN / 2 : BN;  // output channels per tile
+  constexpr int PB = BM >= 128 ? 1 : 2;  // 64-k stages per barrier
+  constexpr int NT = KG * kThreads;
+  constexpr int RING = 3;                 // sets of PB activation stages in LDS
+  constexpr int SB = BM * 128;            // bytes of a stage
+  constexpr int AB = PB * SB;             // bytes of a set
+  constexpr int WB = 64 * 128;            // bytes of a wavefront's code lines
+
+  // per K group: codes [4 wavefronts][64 rows][128 B], activations
+  // [RING][PB][BM][128 B]: 80 KB with KG 1, so that two workgroups share a CU
+  constexpr int GB = 4 * WB + RING * AB;
+  __shared__ __align__(1024) uint8_t smem_all[KG * GB];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6) & 3;
+  const int kgrp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid >> 8);
+  uint8_t* const smem = smem_all + kgrp * GB;
+  uint8_t* const sX = smem + 4 * WB;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem_all + kgrp * GB;
+
+  int g, row0, rows, ntile;
+  if (p.group_offs) {
+    // consecutive workgroups go round-robin to the XCDs: XCD x walks the
+    // m-tiles x, x + 8, ..., all weight tiles of one before the next, so
+    // that an m-tile's activation rows come from one L2
+    const int slot = blockIdx.x / kXcds;
+    ntile = slot % n_tiles;
+    if (!tile_group<BM>(p, slot / n_tiles * kXcds + blockIdx.x % kXcds, g, row0, rows, reinterpret_cast<int*>(smem_all)))
+      return;
+    __syncthreads();  // the group has been read everywhere: the buffers are free
+  } else {
+    int mt;
+    if (!tile_dense(blockIdx.x, m_tiles, n_tiles, mt, ntile)) return;
+    g = 0;
+    row0 = mt * BM;
+    rows = min(BM, p.M - row0);
+  }
+  g = __builtin_amdgcn_readfirstlane(g);
+  const int n0 = ntile * BNO;
+  const int nlim = ACT ? p.N / 2 : p.N;
+  // global weight row of tile row r (gate rows, then up rows with ACT); rows
+  // past the end are clamped (their outputs are never stored)
+  auto wrow_global = [&](int r) {
+    if (ACT) return (r < BN / 2 ? 0 : p.N / 2) + min(n0 + (r % (BN / 2)), nlim - 1);
+    return min(n0 + r, nlim - 1);
+  };
+  // tile row of this wavefront's row m of weight block i
+  auto wrow = [&](int i, int m) { return i * (BN / 2) + 4 * m + wave; };
+
+  // epilogue inputs (loaded now, staged in LDS at the end): token routing
+  // weight and output row; weight-row bias
+  float e_rw = 1.0f, e_bs = 0.0f;
+  int e_yr = 0;
+  if (tid < BM) {
+    const int R = row0 + min(tid, rows - 1);
+    if (p.row_weight) e_rw = bf16_to_f32(p.row_weight[R]);
+    e_yr = p.y_rows ? p.y_rows[R] : R;
+  }
+  if (tid < BN && p.bias) e_bs = p.bias[(int64_t)g * p.bias_gstride + wrow_global(tid)];
+
+  // split-K: the workgroup's stages of 64 k; its K groups take consecutive parts
+  const int NU = p.K / 64;
+  int u0 = (int)((int64_t)NU * blockIdx.z / p.ksplit);
+  int KS = (int)((int64_t)NU * (blockIdx.z + 1) / p.ksplit) - u0;
+  const int sets = cdiv(cdiv(KS, KG), PB);  // barriers that every K group reaches
+  if constexpr (KG == 2) {
+    const int h = (KS + 1) / 2;
+    u0 += kgrp * h;
+    KS = kgrp ? KS - h : h;
+  }
+
+  // ---- activation copies: one instruction = 8 rows x 128 bytes (lane -> row
+  // l >> 3, slot l & 7; the slot of chunk c of row r is c ^ w4_swz(r))
+  constexpr int XI = BM / 32;  // per wavefront and stage; copy j covers rows 32 j .. 32 j + 31
+  const uint8_t* xp[XI];
+#pragma unroll
+  for (int j = 0; j < XI; ++j) {
+    const int r = (wave + 4 * j) * 8 + (lane >> 3);
+    const int R = row0 + min(r, rows - 1);
+    const int ar = p.a_rows ? p.a_rows[R] : R;
+    xp[j] = static_cast<const uint8_t*>(p.a) + (uint64_t)(uint32_t)ar * ((uint64_t)p.lda * 2) +
+            (uint32_t)(((lane & 7) ^ w4_swz(r)) * 16 + u0 * 128);
+  }
+  const uint32_t xdst = lds0 + 4 * WB + wave * 1024;
+
+  // ---- code copies: whole 128-byte lines (256 k) of the wavefront's own 64
+  // rows, 8 rows per instruction. Row bytes are K / 2, any multiple of 32, so
+  // consecutive rows start at up to four different places of a line (phases
+  // of 32 bytes); rows four apart share one, and a wavefront owns every
+  // fourth row. Stage s of the wavefront is quarter (s + ph) % 4 of its line
+  // (s + ph) / 4.
+  const uint8_t* wbase = p.w + (int64_t)g * p.w_gstride;
+  const int rowb = p.K / 2;
+  const int ph = __builtin_amdgcn_readfirstlane(
+      (int)((((uint64_t)reinterpret_cast<uintptr_t>(wbase) + (uint64_t)(uint32_t)wrow_global(wrow(0, 0)) * (uint64_t)p.ldw) >> 5) +
+            (uint64_t)u0) & 3);
+  constexpr int WI = 8;
+  uint32_t roff[WI];
+#pragma unroll
+  for (int j = 0; j < WI; ++j)
+    roff[j] = (uint32_t)wrow_global(wrow(j / 4, (j % 4) * 8 + (lane >> 3))) * (uint32_t)p.ldw;
+  const int wc16 = ((lane & 7) ^ (lane >> 3)) * 16;  // chunk of even j (odd j: the neighbour)
+  const uint32_t wdst = lds0 + wave * WB;
+  auto copy_line = [&](int q) {  // line q of the slice, clamped to the rows
+    const int b = (u0 - ph) * 32 + q * 128;
+    const uint32_t b0 = (uint32_t)min(max(b + wc16, 0), rowb - 16);
+    const uint32_t b1 = (uint32_t)min(max(b + (wc16 ^ 16), 0), rowb - 16);
+#pragma unroll
+    for (int j = 0; j < WI; ++j) w4_copy16(wbase, roff[j] + (j & 1 ? b1 : b0), wdst + j * 1024);
+  };
+
+  // ---- weight scales: lane (row l % 32, half h) of weight block i needs, for
+  // stage u, e8m0 byte 2 u + h of its row; NVFP4: the bf16 pair 4 u + 2 h;
+  // INT4: the bf16 scale of k 64 u + 32 h. Loaded for the four stages of a line.
+  constexpr int kSB = NV || I4 ? 2 : 1;  // bytes per scale
+  constexpr int SW = NV || I4 ? 4 : 2;   // registers per weight block and line
+  const rsrc_t eres = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<void*>(static_cast<const void*>(static_cast<const uint8_t*>(p.w_scale) + (int64_t)g * p.ws_gstride * kSB)),
+      (short)0, (int)std::min<int64_t>((int64_t)p.N * p.ldws * kSB, 0x7fffffff), 0x00020000);
+  const int rl = lane & 31, kh = lane >> 5;
+  uint32_t eoff[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+    eoff[i] = (uint32_t)wrow_global(wrow(i, rl)) * (uint32_t)(p.ldws * kSB) + (NV ? kh * 4 : 0);
+  const int lg = I4 ? (p.wq_group == 32 ? 5 : (p.wq_group == 64 ? 6 : 7)) : 0;  // log2(group)
+  constexpr int NSC = NI * (NV || I4 ? 4 : 2);  // loads
+  uint32_t we[NI][SW], wn[NI][SW];  // the line in use and the next one
+  // scales of stages s .. s + 3 of the slice (those past the end of K: of a
+  // valid stage or zero, for no product). Every call makes NSC loads.
+  auto load_scales = [&](int s) {
+    const int u = u0 + s;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      if constexpr (NV) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          wn[i][k] = __builtin_amdgcn_raw_buffer_load_b32(eres, eoff[i], (uint32_t)min(u + k, NU - 1) * 8u, 0);
+      } else if constexpr (I4) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const uint32_t k0 = (uint32_t)min(u + k, NU - 1) * 64u + (uint32_t)kh * 32u;
+          wn[i][k] = __builtin_amdgcn_raw_buffer_load_b16(eres, eoff[i] + (k0 >> lg) * 2u, 0, 0);
+        }
+      } else {
+        // pairs of stages: 4 bytes, the last stage of an odd K / 64 2 bytes
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+          const int v = min(u + 2 * k, NU - 1);
+          if (v + 1 < NU) wn[i][k] = __builtin_amdgcn_raw_buffer_load_b32(eres, eoff[i], (uint32_t)v * 2u, 0);
+          else wn[i][k] = __builtin_amdgcn_raw_buffer_load_b16(eres, eoff[i], (uint32_t)v * 2u, 0);
+        }
+      }
+    }
+  };
+
+  f32x16 acc[NI][MJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+  // The K pipeline over the first MJE 32-token blocks of the tile (MJ: all
+  // of them); the accumulators of the others keep their zeros.
+  auto pipeline = [&](auto mje_c) {
+    constexpr int MJE = decltype(mje_c)::value;
+    constexpr int XC = PB * MJE;  // copies per set
+    auto copy_x = [&](int ks, int buf) {  // the set of stages ks .. ks + PB - 1
+#pragma unroll
+      for (int h = 0; h < PB; ++h)
+#pragma unroll
+        for (int j = 0; j < MJE; ++j)
+          w4_copy16(xp[j] + min(ks + h, KS - 1) * 128, xdst + buf * AB + h * SB + j * 4096);
+    };
+    uint4 wc[4][NI];  // codes of a line's four stages
+    auto read_line = [&]() {
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const int r = i * 32 + rl;
+          wc[k][i] = *reinterpret_cast<const uint4*>(smem + wave * WB + r * 128 + (((2 * k + kh) ^ w4_swz(r)) * 16));
+        }
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): the codes are in registers
+    };
+    if (KS <= 0) return;
+    const int last_line = (KS - 1 + ph) >> 2;
+    load_scales(0);
+    copy_line(0);
+    copy_x(0, 0);
+    if (KS > PB) copy_x(PB, 1);
+    wait_copies_upto<0>();
+    asm volatile("" ::: "memory");
+    // the first line starts in quarter ph: its scales move to their quarters
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      if constexpr (NV || I4) {
+        const uint32_t e0 = wn[i][0], e1 = wn[i][1], e2 = wn[i][2];
+        if (ph == 1) wn[i][1] = e0, wn[i][2] = e1, wn[i][3] = e2;
+        else if (ph == 2) wn[i][2] = e0, wn[i][3] = e1;
+        else if (ph == 3) wn[i][3] = e0;
+      } else {
+        const uint64_t e = ((uint64_t)wn[i][1] << 32 | wn[i][0]) << (16 * ph);
+        wn[i][0] = (uint32_t)e;
+        wn[i][1] = (uint32_t)(e >> 32);
+      }
+    }
+    int buf = 0;
+    // ---- stages. Per set of PB stages: wait for its activations (the next
+    // set's, and a line and scales copied meanwhile, stay in flight) ->
+    // barrier: they have landed everywhere, and everybody is done with the
+    // previous set -> copy the set after the next into its buffer. At the
+    // start of a line the wavefront takes its codes into registers, which
+    // frees the line buffer for the next line, four stages ahead of its use:
+    // what a workgroup has in flight from memory sets the rate at which it
+    // can stream weights.
+    auto stage = [&](auto k_c, int s) __attribute__((always_inline)) {
+      constexpr int K4 = decltype(k_c)::value;
+      const int line = (s + ph) >> 2;
+      const bool first = PB == 1 || !(s & 1);  // of its set
+      if (first) {
+        // issued after the set's activations: those of the next set, and
+        // scales and codes of a line taken since (in this line's first stage)
+        if (s > 0) {
+          if (s + PB >= KS) wait_copies_upto<0>();
+          else if (K4 != 0 && (PB == 2 || K4 == 1 || s == 1) && line < last_line)
+            wait_copies_upto<XC + NSC + WI>();
+          else wait_copies_upto<XC>();
+        }
+        stage_barrier();
+      } else if (K4 == 0) {
+        // a line that starts inside a set: two sets' activations were copied after it
+        if (s + 3 >= KS) wait_copies_upto<0>();
+        else if (s == 1) wait_copies_upto<XC>();
+        else wait_copies_upto<2 * XC>();
+        asm volatile("" ::: "memory");
+      }
+      if (K4 == 0 || s == 0) {
+        read_line();
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int k = 0; k < SW; ++k) we[i][k] = wn[i][k];
+        if (line < last_line) {
+          load_scales(4 * (line + 1) - ph);
+          asm volatile("" ::: "memory");
+          copy_line(line + 1);
+        }
+      }
+      if (first && s + 2 * PB < KS) copy_x(s + 2 * PB, buf == 0 ? 2 : buf - 1);
+      const uint8_t* sA = sX + buf * AB + (first ? 0 : SB);
+      if (PB == 1 || !first) buf = buf == 2 ? 0 : buf + 1;
+
+      float scale[NI], scale1[NI];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        if constexpr (NV) {  // scale for 16-k steps 0-1, scale1 for 2-3
+          scale[i] = bits_f32(we[i][K4] << 16);
+          scale1[i] = bits_f32(we[i][K4] & 0xffff0000u);
+        } else if constexpr (I4) {
+          scale[i] = bits_f32(we[i][K4] << 16);
+        } else {
+          scale[i] = e8m0_to_f32(we[i][K4 / 2] >> ((K4 & 1) * 16 + 8 * kh));
+        }
+      }
+      uint4 xa[2][MJE];
+      auto read_x = [&](int q) {
+#pragma unroll
+        for (int j = 0; j < MJE; ++j) {
+          const int r = j * 32 + rl;
+          xa[q & 1][j] = *reinterpret_cast<const uint4*>(sA + r * 128 + (((kh * 4 + q) ^ w4_swz(r)) * 16));
+        }
+      };
+      read_x(0);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        if (q < 3) read_x(q + 1);
+        bf16x8 wv[NI];
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          // dword q of the lane's 16 code bytes feeds 16-k step q
+          const uint4 c4 = wc[K4][i];
+          const uint32_t d = q == 0 ? c4.x : (q == 1 ? c4.y : (q == 2 ? c4.z : c4.w));
+          if constexpr (NV) wv[i] = as_bf16x8_u4(nvfp4x8_to_bf16(d, q < 2 ? scale[i] : scale1[i]));
+          else if constexpr (I4) wv[i] = as_bf16x8_u4(int4x8_to_bf16(d, scale[i]));
+          else wv[i] = w4_expand(d, scale[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < MJE; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv[i], as_bf16x8_u4(xa[q & 1][j]), acc[i][j], 0, 0, 0);
+      }
+    };
+    for (int s = -ph; s < KS; s += 4) {
+      if (s >= 0) stage(std::integral_constant<int, 0>{}, s);
+      if (s + 1 >= 0 && s + 1 < KS) stage(std::integral_constant<int, 1>{}, s + 1);
+      if (s + 2 >= 0 && s + 2 < KS) stage(std::integral_constant<int, 2>{}, s + 2);
+      if (s + 3 >= 0 && s + 3 < KS) stage(std::integral_constant<int, 3>{}, s + 3);
+    }
+  };
+  // A tile with few valid tokens -- a routed expert's last tile -- copies and
+  // multiplies its occupied 32-token blocks only.
+  const int rows_u = __builtin_amdgcn_readfirstlane(rows);
+  if constexpr (MJ == 4) {
+    if (rows_u <= 32) pipeline(std::integral_constant<int, 1>{});
+    else if (rows_u <= 64) pipeline(std::integral_constant<int, 2>{});
+    else if (rows_u <= 96) pipeline(std::integral_constant<int, 3>{});
+    else pipeline(std::integral_constant<int, 4>{});
+  } else if constexpr (MJ == 2) {
+    if (rows_u <= 32) pipeline(std::integral_constant<int, 1>{});
+    else pipeline(std::integral_constant<int, 2>{});
+  } else {
+    pipeline(std::integral_constant<int, MJ>{});
+  }
+
+  if constexpr (KG == 2)
+    for (int b = cdiv(KS, PB); b < sets; ++b) stage_barrier();
+
+  // ---- epilogue: per 32-token block, the workgroup's f32 sums in LDS
+  // ([32 tokens][256 tile rows], row n of token t at n ^ 4 (t % 16); the
+  // second K group adds to the first's), then 8 output channels of a token
+  // per thread
+  __syncthreads();  // every wavefront is done with the stage buffers
+  float* reg = reinterpret_cast<float*>(smem_all);
+  float* s_rw = reinterpret_cast<float*>(smem_all + 4 * WB);
+  float* s_bs = s_rw + BM;
+  int* s_yr = reinterpret_cast<int*>(s_bs + BN);
+  static_assert(32 * BN * 4 <= 4 * WB && (2 * BM + BN) * 4 <= RING * AB, "epilogue regions");
+  if (tid < BM) {
+    s_rw[tid] = e_rw;
+    s_yr[tid] = e_yr;
+  }
+  if (tid < BN) s_bs[tid] = e_bs;
+  const bool vec_ok = ((p.ldy & 7) == 0) && ((reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
+  const bool has_bias = p.bias != nullptr;
+#pragma unroll
+  for (int j = 0; j < MJ; ++j) {
+    if (j * 32 >= rows_u) break;
+    if (j) __syncthreads();  // the previous block has been read
+#pragma unroll
+    for (int kk = 0; kk < KG; ++kk) {
+      if (kgrp == kk) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) {
+            const int m = 8 * (r / 4) + 4 * kh + (r % 4);  // MFMA row of register r
+            float& d = reg[rl * BN + (wrow(i, m) ^ (4 * (rl & 15)))];
+            d = kk ? d + acc[i][j][r] : acc[i][j][r];
+          }
+      }
+      __syncthreads();
+    }
+    auto quad = [&](int t, int n) {
+      return *reinterpret_cast<const float4*>(reg + t * BN + (n ^ (4 * (t & 15))));
+    };
+    if (p.ksplit > 1) {
+      // raw sums to the f32 workspace [ksplit][M][N]; the finishing kernel
+      // adds the slices in order and runs the epilogue
+      float* plane = p.partial + (int64_t)blockIdx.z * p.M * p.N;
+      for (int e = tid; e < 32 * BN / 4; e += NT) {
+        const int t = e / (BN / 4), r = (e % (BN / 4)) * 4;
+        const int tr = j * 32 + t;
+        const int c = n0 + (ACT ? r % (BN / 2) : r);  // output channel of the quad
+        if (tr >= rows || c >= nlim) continue;
+        const float4 v = quad(t, r);
+        float* dst = plane + (int64_t)(row0 + tr) * p.N + (ACT && r >= BN / 2 ? p.N / 2 : 0) + c;
+        if (c + 4 <= nlim && (p.N & 3) == 0 && (!ACT || (p.N & 7) == 0)) {
+          *reinterpret_cast<float4*>(dst) = v;
+        } else {
+          const float f[4] = {v.x, v.y, v.z, v.w};
+          for (int k = 0; k < 4 && c + k < nlim; ++k) dst[k] = f[k];
+        }
+      }
+      continue;
+    }
+    for (int e = tid; e < 32 * (BNO / 8); e += NT) {
+      const int t = e / (BNO / 8), c = (e % (BNO / 8)) * 8;  // token of the block, first tile channel
+      const int tr = j * 32 + t;
+      if (tr >= rows || n0 + c >= nlim) continue;
+      const float4 g0 = quad(t, c), g1 = quad(t, c + 4);
+      const float vg[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+      float vu[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      if (ACT) {
+        const float4 h0 = quad(t, BN / 2 + c), h1 = quad(t, BN / 2 + c + 4);
+        vu[0] = h0.x; vu[1] = h0.y; vu[2] = h0.z; vu[3] = h0.w;
+        vu[4] = h1.x; vu[5] = h1.y; vu[6] = h1.z; vu[7] = h1.w;
+      }
+      const float rwt = s_rw[tr];
+      uint32_t packed[4];
+#pragma unroll
+      for (int k = 0; k < 8; k += 2) {
+        float o2[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          float v = vg[k + h];
+          if (has_bias) v += s_bs[c + k + h];
+          if (ACT) {
+            float u = vu[k + h];
+            if (has_bias) u += s_bs[BN / 2 + c + k + h];
+            v = qmoe_act(p.act, v, u, p.act_p0, p.act_p1);
+          }
+          o2[h] = v * rwt;
+        }
+        packed[k / 2] = (uint32_t)f32_to_bf16(o2[0]) | ((uint32_t)f32_to_bf16(o2[1]) << 16);
+      }
+      uint16_t* dst = p.y + (int64_t)s_yr[tr] * p.ldy + n0 + c;
+      if (vec_ok && n0 + c + 8 <= nlim) {
+        *reinterpret_cast<uint4*>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+      } else {
+        for (int k = 0; k < 8 && n0 + c + k < nlim; ++k) dst[k] = (uint16_t)(packed[k / 2] >> ((k & 1) * 16));
+      }
+    }
+  }
+}
+
+// The wavefronts split the 256 weight rows (each expands its own 64 rows
+// once per stage and reuses them for all BM tokens); WN = 4 always.
+template <int BM>
+struct W4Shape {
+  static constexpr int WN = 4;                  // wavefronts along weight rows
+  static constexpr int WM = 1;                  // along tokens
+  static constexpr int TN = kW4BN / WN;         // weight rows per wavefront
+  static constexpr int TM = BM / WM;            // tokens per wavefront
+  static constexpr int NI = TN / 32;
+  static constexpr int MJ = TM / 32;
+  static_assert(NI >= 1 && MJ >= 1, "tile too small");
+};
+
+// Short under-filled dense problems of the costlier formats (1 NVFP4, 2 INT4;
+// w4_ring below has the rule): one workgroup per tile whose stages of 64 k --
+// activations, codes and scales alike -- run through a ring of four, copied
+// four stages ahead, with the operand reads and copies of a stage spread
+// over its MFMAs. It spends fewer instructions per stage than the line
+// pipeline above, and with one workgroup per CU that is what counts: NVFP4 K
+// 2880, N 5760 at 128 / 203 tokens 23.4 / 28.1 us against 26.0 / 32.0.
 template <int BM, bool ACT, int FMT>
-__global__ __launch_bounds__(kThreads) void w4_gemm_kernel(const GemmParams p, int m_tiles, int n_tiles) {
+__global__ __launch_bounds__(kThreads) void w4_ring_kernel(const GemmParams p, int m_tiles, int n_tiles) {
   constexpr bool NV = FMT == 1, I4 = FMT == 2;
   using S = W4Shape<BM>;
   constexpr int BN = kW4BN;
@@ -94,7 +552,6 @@ __global__ __launch_bounds__(kThreads) void w4_gemm_kernel(const GemmParams p, i
   // four LDS stages of 64 k: activations [BM][128 B], codes [BN][32 B]
   __shared__ __align__(1024) uint8_t sA0[BM * 128], sA1[BM * 128], sA2[BM * 128], sA3[BM * 128];
   __shared__ __align__(1024) uint8_t sW0[BN * 32], sW1[BN * 32], sW2[BN * 32], sW3[BN * 32];
-  __shared__ int s_info[4];
   __shared__ float s_sx[BM], s_rw[BM], s_ws[BN], s_bs[BN];
   __shared__ int s_yr[BM];
 
@@ -103,10 +560,7 @@ __global__ __launch_bounds__(kThreads) void w4_gemm_kernel(const GemmParams p, i
   const int wn = wave % S::WN, wm = wave / S::WN;
 
   int g, row0, rows, ntile;
-  if (p.group_offs) {
-    if (!tile_group<BM>(p, blockIdx.y, g, row0, rows, s_info)) return;
-    ntile = blockIdx.x;
-  } else {
+  {
     int mt;
     if (!tile_dense(blockIdx.x, m_tiles, n_tiles, mt, ntile)) return;
     g = 0;
@@ -140,7 +594,8 @@ __global__ __launch_bounds__(kThreads) void w4_gemm_kernel(const GemmParams p, i
   // lane (row l % 32, half h) of weight block i needs e8m0 byte 2*stage + h
   // of its row (NVFP4: bf16 scales 4*stage + 2h and + 1, one 4-byte load;
   // INT4: bf16 scale (64*stage + 32h) / group).
-  constexpr int kSB = NV || I4 ? 2 : 1;  // bytes per scale
+  static_assert(NV || I4, "bf16 scales");
+  constexpr int kSB = 2;  // bytes per scale
   constexpr int XI = BM / 32;  // activation copies per wavefront
   constexpr int WI = 2;        // code copies per wavefront
   const uint8_t* xbase = static_cast<const uint8_t*>(p.a);
@@ -174,7 +629,7 @@ __global__ __launch_bounds__(kThreads) void w4_gemm_kernel(const GemmParams p, i
   uint32_t eoff[NI];
 #pragma unroll
   for (int i = 0; i < NI; ++i)
-    eoff[i] = (uint32_t)wrow_global(wrow(i) + rl) * (uint32_t)(p.ldws * kSB) + (NV ? kh * 4 : (I4 ? 0 : kh));
+    eoff[i] = (uint32_t)wrow_global(wrow(i) + rl) * (uint32_t)(p.ldws * kSB) + (NV ? kh * 4 : 0);
   const int lg = I4 ? (p.wq_group == 32 ? 5 : (p.wq_group == 64 ? 6 : 7)) : 0;  // log2(group)
   uint32_t we[4][NI];  // scales of the stages in flight (stage s in set s % 4)
   auto copy_stage = [&](uint8_t* dA, uint8_t* dW, int e, int ks) {
@@ -196,11 +651,9 @@ __global__ __launch_bounds__(kThreads) void w4_gemm_kernel(const GemmParams p, i
     for (int i = 0; i < NI; ++i) {
       if constexpr (NV) {
         we[e][i] = __builtin_amdgcn_raw_buffer_load_b32(eres, eoff[i], st * 8u, 0);
-      } else if constexpr (I4) {
+      } else {
         const uint32_t gi = (st * 64u + (uint32_t)kh * 32u) >> lg;  // group of the lane's 32 k
         we[e][i] = __builtin_amdgcn_raw_buffer_load_b16(eres, eoff[i] + gi * 2u, 0, 0);
-      } else {
-        we[e][i] = __builtin_amdgcn_raw_buffer_load_b8(eres, eoff[i], st * 2u, 0);
       }
     }
   };
@@ -245,10 +698,8 @@ __global__ __launch_bounds__(kThreads) void w4_gemm_kernel(const GemmParams p, i
         if constexpr (NV) {
           scale[i] = bits_f32(eb[i] << 16);
           scale1[i] = bits_f32(eb[i] & 0xffff0000u);
-        } else if constexpr (I4) {
-          scale[i] = bits_f32(eb[i] << 16);
         } else {
-          scale[i] = e8m0_to_f32(eb[i]);
+          scale[i] = bits_f32(eb[i] << 16);
         }
       }
 #pragma unroll
@@ -258,8 +709,7 @@ __global__ __launch_bounds__(kThreads) void w4_gemm_kernel(const GemmParams p, i
         for (int i = 0; i < NI; ++i) {
           const uint32_t d = q == 0 ? wc[t][i].x : (q == 1 ? wc[t][i].y : (q == 2 ? wc[t][i].z : wc[t][i].w));
           if constexpr (NV) wv[i] = as_bf16x8_u4(nvfp4x8_to_bf16(d, q < 2 ? scale[i] : scale1[i]));
-          else if constexpr (I4) wv[i] = as_bf16x8_u4(int4x8_to_bf16(d, scale[i]));
-          else wv[i] = w4_expand(d, scale[i]);
+          else wv[i] = as_bf16x8_u4(int4x8_to_bf16(d, scale[i]));
         }
 #pragma unroll
         for (int i = 0; i < NI; ++i)
@@ -354,34 +804,47 @@ __global__ __launch_bounds__(kThreads) void w4_gemm_kernel(const GemmParams p, i
                                         n0, nlim, rows, wn, wm, lane);
 }
 
-template <int BM, bool ACT, int FMT>
+template <int BM, int KG, bool ACT, int FMT>
 void w4_launch_shape(const GemmParams& p, hipStream_t st) {
   const int nout = ACT ? p.N / 2 : p.N;
   const int n_tiles = cdiv(nout, ACT ? kW4BN / 2 : kW4BN);
   const unsigned ks = (unsigned)std::max(1, p.ksplit);
-  if (p.group_offs) {
-    const int m_tiles = cdiv(p.M, BM) + std::min(p.slots, p.M);
-    hipLaunchKernelGGL((w4_gemm_kernel<BM, ACT, FMT>), dim3(n_tiles, m_tiles, ks), dim3(kThreads), 0, st, p,
-                       m_tiles, n_tiles);
-  } else {
-    const int m_tiles = cdiv(p.M, BM);
-    const int grid = cdiv(m_tiles * n_tiles, kXcds) * kXcds;
-    hipLaunchKernelGGL((w4_gemm_kernel<BM, ACT, FMT>), dim3(grid, 1, ks), dim3(kThreads), 0, st, p, m_tiles,
-                       n_tiles);
-  }
+  const int m_tiles = p.group_offs ? cdiv(cdiv(p.M, BM) + std::min(p.slots, p.M), kXcds) * kXcds : cdiv(p.M, BM);
+  const int grid = p.group_offs ? m_tiles * n_tiles : cdiv(m_tiles * n_tiles, kXcds) * kXcds;
+  hipLaunchKernelGGL((w4_gemm_kernel<BM, KG, ACT, FMT>), dim3(grid, 1, ks), dim3(KG * kThreads), 0, st, p, m_tiles,
+                     n_tiles);
+}
+
+template <int BM, int KG, int FMT>
+void w4_launch_act(const GemmParams& p, hipStream_t st) {
+  if (p.act != QA_NONE) w4_launch_shape<BM, KG, true, FMT>(p, st);
+  else w4_launch_shape<BM, KG, false, FMT>(p, st);
+}
+
+template <int BM, int KG>
+void w4_launch_fmt(const GemmParams& p, int fmt, hipStream_t st) {
+  if (fmt == 1) w4_launch_act<BM, KG, 1>(p, st);
+  else if (fmt == 2) w4_launch_act<BM, KG, 2>(p, st);
+  else w4_launch_act<BM, KG, 0>(p, st);
 }
 
 template <int BM, int FMT>
-void w4_launch_act(const GemmParams& p, hipStream_t st) {
-  if (p.act != QA_NONE) w4_launch_shape<BM, true, FMT>(p, st);
-  else w4_launch_shape<BM, false, FMT>(p, st);
+void w4_launch_ring(const GemmParams& p, hipStream_t st) {
+  const bool act = p.act != QA_NONE;
+  const int n_tiles = cdiv(act ? p.N / 2 : p.N, act ? kW4BN / 2 : kW4BN), m_tiles = cdiv(p.M, BM);
+  const dim3 grid(cdiv(m_tiles * n_tiles, kXcds) * kXcds, 1, (unsigned)std::max(1, p.ksplit));
+  if (act) hipLaunchKernelGGL((w4_ring_kernel<BM, true, FMT>), grid, dim3(kThreads), 0, st, p, m_tiles, n_tiles);
+  else hipLaunchKernelGGL((w4_ring_kernel<BM, false, FMT>), grid, dim3(kThreads), 0, st, p, m_tiles, n_tiles);
 }
 
-template <int BM>
-void w4_launch_fmt(const GemmParams& p, int fmt, hipStream_t st) {
-  if (fmt == 1) w4_launch_act<BM, 1>(p, st);
-  else if (fmt == 2) w4_launch_act<BM, 2>(p, st);
-  else w4_launch_act<BM, 0>(p, st);
+// Dense NVFP4 / INT4 problems of at most 256 tokens whose 64-token tiles would
+// leave half of the CUs idle and whose K is too short to split: the ring
+// kernel. Measured on MI355X, NVFP4: K 2880, N 5760 at 128 / 203 tokens 23.4 /
+// 28.1 us against 26.0 / 32.0; with 224 such tiles (N 14336, K 4096, 203
+// tokens) the line pipeline takes 52.5 us against 70.9, with K 14336, N 4096
+// 52.7 against 136.
+bool w4_ring(const GemmParams& p, int fmt, int n_tiles) {
+  return fmt != 0 && !p.group_offs && p.M <= 256 && p.K <= 4096 && cdiv(p.M, 64) * n_tiles < 128;
 }
 
 }  // namespace
@@ -408,51 +871,58 @@ bool qmoe_w4_plan(const GemmParams& p, int fmt, int* bm_out, int* ksplit_out, in
     return false;
   const int nout = p.act != QA_NONE ? p.N / 2 : p.N;
   const int n_tiles = cdiv(nout, p.act != QA_NONE ? kW4BN / 2 : kW4BN);
-  int bm = 32;
+  int bm = 64, ksplit = 1;
   const char* env = getenv("QMOE_W4_BM");  // tuning knob
   if (env && (atoi(env) == 128 || atoi(env) == 64 || atoi(env) == 32)) {
-    bm = atoi(env);
+    bm = p.group_offs && atoi(env) == 32 ? 64 : atoi(env);
   } else if (p.group_offs) {
-    // measured on MI355X (GPT-OSS MoE, 128 experts): 64-token tiles up to
-    // ~96 rows per routed expert (32-token tiles lose ~25% at 32 rows), 128
-    // above
-    const int avg = std::max(1, p.M / std::max(1, std::min(p.slots, p.M)));
-    bm = avg > 96 ? 128 : 64;
-  } else {
-    // measured on MI355X (K 2880, N 5760): 128-token tiles once they fill the
-    // CUs, else 64 with a K split (32-token tiles are slower at every M)
-    bm = (int64_t)cdiv(p.M, 128) * n_tiles >= 200 ? 128 : 64;
-  }
-  const int m_tiles0 = p.group_offs ? cdiv(p.M, bm) + std::min(p.slots, p.M) : cdiv(p.M, bm);
-  if (p.group_offs && m_tiles0 > 65535) return false;
-  // dense problems with fewer than ~200 tiles split K (every slice keeps at
-  // least 8 stages)
-  int ksplit = 1;
-  if (!p.group_offs) {
-    const int tiles = m_tiles0 * n_tiles;
-    if (tiles < 200) ksplit = std::min(cdiv(256, tiles), std::max(1, (p.K / 64) / 8));
-  }
-  // e2m1 (MXFP4 / NVFP4) dense problems too small for 200 128-token tiles:
-  // measured on MI355X (K 2880, N 5760), 32-token tiles with a K split that
-  // shrinks as the tokens grow (MXFP4 64 tokens: 15.5 vs 20.0 us; 256: 25.5
-  // vs 32.2 us). INT4's costlier expansion keeps the larger tiles.
-  if (!p.group_offs && fmt != 2 && !env && (int64_t)cdiv(p.M, 128) * n_tiles < 200 && p.M <= 512) {
-    if (p.M <= 256) {
+    // measured on MI355X (GPT-OSS MoE, 128 experts, MXFP4): 64 rows per
+    // routed expert 797 us in 64-token tiles (half of the experts need a
+    // second one) and 696 in 128-token tiles, 32 rows 518 and 532
+    bm = p.M / std::max(1, std::min(p.slots, p.M)) > 40 ? 128 : 64;
+  } else if (w4_ring(p, fmt, n_tiles)) {
+    // (tile, split) measured best: NVFP4 32-token tiles, 4 slices up to 64
+    // tokens, 2 up to 128; INT4's costlier expansion keeps larger tiles
+    const int tiles = cdiv(p.M, 64) * n_tiles;
+    if (fmt == 1) {
       bm = 32;
       ksplit = p.M <= 64 ? 4 : (p.M <= 128 ? 2 : 1);
+    } else if (p.M <= 128) {
+      ksplit = std::min(cdiv(256, tiles), std::max(1, (p.K / 64) / 8));
     } else {
-      bm = 64;
-      ksplit = 1;
+      bm = 128;
+      ksplit = 4;
     }
     ksplit = std::max(1, std::min(ksplit, p.K / 64));
-  }
-  // INT4 from 129 to 512 tokens in the same regime: 128-token tiles split
-  // 4 / 2 ways (measured on MI355X, K 2880, N 5760: 256 tokens 33.9 vs 38.2
-  // us, 512 tokens 45.6 vs 48.1 us)
-  if (!p.group_offs && fmt == 2 && !env && (int64_t)cdiv(p.M, 128) * n_tiles < 200 && p.M > 128 && p.M <= 512) {
+  } else if (cdiv(p.M, 128) * n_tiles < 256) {
+    // Fewer than 256 128-token tiles: two K groups of wavefronts per
+    // workgroup, one workgroup per CU, in the largest tiles that put at least
+    // 130 workgroups on the 256 CUs, with K in up to 4 slices of at least 28
+    // stages; else 32-token tiles with slices of at least 16. Measured on
+    // MI355X (MXFP4): K 2880, N 5760 at 203 / 512 / 1024 tokens 19.3 / 29.5 /
+    // 47.5 us (32-, 64-, 128-token tiles; the others 26 / 37 / 57), K 14336,
+    // N 4096 at 203 / 512 42.1 / 69.5 (64-, 128-token tiles, 4 slices)
+    const int nu = p.K / 64;
+    bool found = false;
+    for (int b : {128, 64, 32}) {
+      const int t = cdiv(p.M, b) * n_tiles;
+      const int k = std::max(1, std::min({256 / std::max(t, 1), 4, nu / 28}));
+      if (t <= 256 && t * k >= 130) {
+        bm = b;
+        ksplit = k;
+        found = true;
+        break;
+      }
+    }
+    if (!found) {
+      bm = 32;
+      ksplit = std::max(1, std::min({256 / std::max(1, cdiv(p.M, 32) * n_tiles), 4, nu / 16}));
+    }
+  } else {
     bm = 128;
-    ksplit = std::max(1, std::min(p.M <= 256 ? 4 : 2, p.K / 64));
   }
+  const int m_tiles0 = p.group_offs ? cdiv(p.M, bm) + std::min(p.slots, p.M) : cdiv(p.M, bm);
+  if ((int64_t)m_tiles0 * n_tiles > (1 << 30)) return false;
   const char* ks_env = getenv("QMOE_W4_KSPLIT");  // tuning knob
   if (ks_env && atoi(ks_env) > 0) ksplit = std::max(1, std::min(atoi(ks_env), p.K / 64));
   *bm_out = bm;
@@ -472,10 +942,20 @@ int qmoe_w4_launch(GemmParams p, int fmt, void* workspace, int64_t ws_bytes, hip
     if (!workspace || ws_bytes < need) return QMOE_ERR_WORKSPACE;
     p.partial = static_cast<float*>(workspace);
   }
-  switch (bm) {
-    case 128: w4_launch_fmt<128>(p, fmt, st); break;
-    case 64: w4_launch_fmt<64>(p, fmt, st); break;
-    default: w4_launch_fmt<32>(p, fmt, st); break;
+  const int n_tiles = cdiv(p.act != QA_NONE ? p.N / 2 : p.N, p.act != QA_NONE ? kW4BN / 2 : kW4BN);
+  if (w4_ring(p, fmt, n_tiles)) {
+    if (fmt == 1) w4_launch_ring<32, 1>(p, st);
+    else if (bm == 128) w4_launch_ring<128, 2>(p, st);
+    else w4_launch_ring<64, 2>(p, st);
+  } else if (bm == 128) {
+    // two K groups of wavefronts per workgroup where one workgroup per CU is all there is
+    if (p.group_offs || cdiv(p.M, 128) * n_tiles * ksplit > 256) w4_launch_fmt<128, 1>(p, fmt, st);
+    else w4_launch_fmt<128, 2>(p, fmt, st);
+  } else if (bm == 64) {
+    if (p.group_offs) w4_launch_fmt<64, 1>(p, fmt, st);
+    else w4_launch_fmt<64, 2>(p, fmt, st);
+  } else {
+    w4_launch_fmt<32, 2>(p, fmt, st);
   }
   if (ksplit > 1) {
     const int nout = p.act != QA_NONE ? p.N / 2 : p.N;
