@@ -18,6 +18,8 @@ int qmoe_tiled_launch(int kind, GemmParams p, void* workspace, int64_t ws_bytes,
 int qmoe_tiled_plan(int kind, const GemmParams& p, int* tile, int* ksplit, int64_t* ws_bytes);
 bool qmoe_f8_plan(const GemmParams& p, bool blk, int* bm_out, int* ksplit_out, int64_t* ws_bytes, int* bn_out);
 int qmoe_f8_launch(GemmParams p, bool blk, void* workspace, int64_t ws_bytes, hipStream_t st);
+int qmoe_t8_plan(const GemmParams& p, bool f8);
+int qmoe_t8_launch(GemmParams p, bool f8, hipStream_t st);
 int qmoe_mx_plan(const GemmParams& p);
 int qmoe_mx_launch(GemmParams p, hipStream_t st);
 bool qmoe_f8_persistent(const GemmParams& p, bool blk);
@@ -225,6 +227,7 @@ enum Path {
   kPathSkinnyDyn = 8,     // weight streaming with the per-row activation quantization inside
   kPathF8Narrow = 9,      // 1-byte x 1-byte tiles of 128 weight rows
   kPathSkinnyRows = 10,   // weight streaming, one slice of rows per grid.z index
+  kPathT8 = 11,           // eight-wavefront tiles (block-scaled e4m3, bf16 x bf16)
 };
 
 // Dense problems of a few dozen rows can stream the weights once per slice
@@ -352,6 +355,10 @@ int qmoe_route_of(const qmoe_gemm_desc* d, GemmParams& p, QmoeRoute* r) {
     int bm = 0, ks = 1;
     int64_t ws = 0;
     int bn = 256;
+    if ((kind == QK_W16A16 || (kind == QK_W8A8_BLK && use_f8(d))) && (bm = qmoe_t8_plan(p, kind == QK_W8A8_BLK))) {
+      *r = QmoeRoute{kPathT8, bm, 1, 0};
+      return QMOE_OK;
+    }
     if (use_f8(d) && qmoe_f8_plan(p, kind == QK_W8A8_BLK, &bm, &ks, &ws, &bn)) {
       const int path = bn == 128 ? kPathF8Narrow
                                  : (qmoe_f8_persistent(p, kind == QK_W8A8_BLK) ? kPathF8Persistent : kPathF8);
@@ -420,6 +427,7 @@ int qmoe_run_route(const qmoe_gemm_desc* d, const QmoeRoute& r, GemmParams p, vo
     case kPathF8Narrow:
     case kPathF8Persistent: return qmoe_f8_launch(p, kind == QK_W8A8_BLK, workspace, ws_bytes, stream);
     case kPathW4: return qmoe_w4_launch(p, w4_fmt(d), workspace, ws_bytes, stream);
+    case kPathT8: return qmoe_t8_launch(p, kind == QK_W8A8_BLK, stream);
     case kPathTiled: return qmoe_tiled_launch(kind, p, workspace, ws_bytes, stream);
     case kPathMx:
     case kPathMxTiles: return qmoe_mx_launch(p, stream);

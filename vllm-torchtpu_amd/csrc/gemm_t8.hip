@@ -1,0 +1,460 @@
+// Tiles of eight wavefronts (one workgroup per CU, two wavefronts per SIMD):
+// block-scaled FP8 (QK_W8A8_BLK, e4m3 codes: 128 x 128 weight tiles or the
+// grouped matmul's per-channel weights, activation scales per 128 or 512
+// columns) and bf16 x bf16 (QK_W16A16), dense or grouped.
+//
+//  * What bounds it: the matrix cores with the vector ALU and the operand
+//    reads beside them. A block-scaled tile adds every 128-k block's sums,
+//    scaled, to its accumulators: 16 FMAs per 32 x 32 block against two MFMAs
+//    of 64 cycles. With one wavefront per SIMD (gemm_f8.hip) these alternate
+//    and the second accumulator set in AGPRs costs another 16 moves; with two
+//    wavefronts of at most 256 VGPRs the MFMAs write VGPRs directly, and one
+//    wavefront scales while the other multiplies.
+//  * Output tile BM tokens x 256 weight rows; wavefront (wn, wm), wn < 4,
+//    wm < 2, owns 64 weight rows (two 32-row blocks) and the 32-token blocks
+//    wm, wm + 2, ..., so that a tile with few tokens loads both halves alike.
+//    Measured (DeepSeek-V3 gate_up, K 7168, N 18432, 2048 / 8192 tokens): 389 /
+//    1497 -> 354 / 1246 us; routed experts (256, top 8), 2048 tokens: 2659 ->
+//    2356 us; bf16 K 4096, N 6144, 1024 tokens 84 -> 62 us. What is left is
+//    the copies: 64 KB per stage of 2048 MFMA cycles, where the L2 delivers
+//    about 29 bytes per cycle and CU.
+//  * Stages of 128 bytes of every row (128 e4m3 / 64 bf16 values), copied
+//    straight into a ring of LDS stages (two of 64 KB for 256 tokens, three of
+//    48 KB for 128); one barrier per stage.
+//  * The epilogue takes 64 tokens at a time through LDS (32 x 256 f32 sums per
+//    token block) and finishes 8 channels of a token per thread.
+
+#include <algorithm>
+#include <cstdlib>
+#include <type_traits>
+
+#include "gemm_tile.h"
+#include "stream_load.h"
+
+namespace {
+
+constexpr int kT8Threads = 512;
+constexpr int kT8BN = 256;
+
+__device__ __forceinline__ int t8_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+
+// Wait until at most n vector-memory operations are outstanding, n < 12 known
+// at run time (wave-uniform)
+__device__ __forceinline__ void t8_wait(int n) {
+  switch (n) {
+    case 4: wait_copies_upto<4>(); break;
+    case 5: wait_copies_upto<5>(); break;
+    case 6: wait_copies_upto<6>(); break;
+    case 7: wait_copies_upto<7>(); break;
+    default: wait_copies_upto<0>(); break;
+  }
+}
+
+// F8: block-scaled e4m3; else bf16. WPC (F8): one weight scale per weight row,
+// applied in the epilogue, instead of one per 128 x 128 tile.
+template <bool F8, int BM, bool ACT, bool WPC>
+__global__ __launch_bounds__(kT8Threads, 2) void t8_gemm_kernel(const GemmParams p, int m_tiles, int n_tiles) {
+  constexpr int BN = kT8BN, BNO = ACT ? BN / 2 : BN;
+  constexpr int NI = 2, MJ = BM / 64;            // 32-row weight blocks, 32-token blocks per wavefront
+  constexpr int RING = BM > 128 ? 2 : 3;
+  constexpr int WB = BN * 128, XB = BM * 128;    // bytes of a stage
+  constexpr int STG = WB + XB + (F8 ? BM * 4 : 0);
+  __shared__ __align__(1024) uint8_t smem[RING * STG];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem;
+
+  const int tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wn = wave & 3, wm = wave >> 2;
+
+  int g, row0, rows, ntile;
+  if (p.group_offs) {
+    // XCD x walks the m-tiles x, x + 8, ..., all weight tiles of one before
+    // the next (an m-tile's activation rows come from one L2)
+    const int slot = blockIdx.x / kXcds;
+    ntile = slot % n_tiles;
+    if (!tile_group<BM>(p, slot / n_tiles * kXcds + blockIdx.x % kXcds, g, row0, rows, reinterpret_cast<int*>(smem)))
+      return;
+    __syncthreads();  // the group has been read everywhere: the buffers are free
+  } else {
+    int mt;
+    if (!tile_dense(blockIdx.x, m_tiles, n_tiles, mt, ntile)) return;
+    g = 0;
+    row0 = mt * BM;
+    rows = min(BM, p.M - row0);
+  }
+  g = __builtin_amdgcn_readfirstlane(g);
+  const int rows_u = __builtin_amdgcn_readfirstlane(rows);
+  const int n0 = ntile * BNO;
+  const int nlim = ACT ? p.N / 2 : p.N;
+  // global weight row of tile row r (gate rows, then up rows with ACT); rows
+  // past the end are clamped (their outputs are never stored). With ACT a
+  // wavefront's first block holds gate rows and its second the matching up
+  // rows.
+  auto wrow_global = [&](int r) {
+    if (ACT) return (r < BN / 2 ? 0 : p.N / 2) + min(n0 + (r % (BN / 2)), nlim - 1);
+    return min(n0 + r, nlim - 1);
+  };
+  auto wrow = [&](int i) { return ACT ? i * (BN / 2) + wn * 32 : wn * 64 + i * 32; };
+
+  // epilogue inputs (loaded now, staged in LDS at the end)
+  float e_rw = 1.0f, e_bs = 0.0f, e_ws = 1.0f;
+  int e_yr = 0;
+  if (tid < BM) {
+    const int R = row0 + min(tid, rows - 1);
+    if (p.row_weight) e_rw = bf16_to_f32(p.row_weight[R]);
+    e_yr = p.y_rows ? p.y_rows[R] : R;
+  }
+  if (tid < BN) {
+    if (p.bias) e_bs = p.bias[(int64_t)g * p.bias_gstride + wrow_global(tid)];
+    if constexpr (F8 && WPC) e_ws = static_cast<const float*>(p.w_scale)[(int64_t)g * p.ws_gstride + wrow_global(tid)];
+  }
+
+  // ---- copies: one instruction = 8 rows x 128 bytes (lane -> row l >> 3, slot
+  // l & 7; the slot of chunk c of row r is c ^ t8_swz(r)); wavefront w copies
+  // the row groups w, w + 8, ... of both operands. Activation row groups past
+  // the tile's rows are left out.
+  constexpr int WI = BN / 64, XI = BM / 64;
+  const uint64_t ab = F8 ? 1 : 2;
+  const uint8_t* wbase = p.w + (int64_t)g * p.w_gstride;
+  const int cchunk = ((lane & 7) ^ ((lane >> 3) ^ (wave & 1))) * 16;
+  uint32_t woff[WI];
+#pragma unroll
+  for (int j = 0; j < WI; ++j)
+    woff[j] = (uint32_t)wrow_global((wave + 8 * j) * 8 + (lane >> 3)) * (uint32_t)p.ldw + (uint32_t)cchunk;
+  const uint8_t* xp[XI];
+  int nx = 0;
+#pragma unroll
+  for (int j = 0; j < XI; ++j) {
+    const int r = (wave + 8 * j) * 8 + (lane >> 3);
+    const int R = row0 + min(r, rows - 1);
+    const int ar = p.a_rows ? p.a_rows[R] : R;
+    xp[j] = static_cast<const uint8_t*>(p.a) + (uint64_t)(uint32_t)ar * ((uint64_t)p.lda * ab) + (uint32_t)cchunk;
+    nx += (wave + 8 * j) * 8 < rows_u ? 1 : 0;
+  }
+  // F8: the activation scales of a stage, 64 tokens per wavefront
+  const float* sp = p.a_scale;
+  const bool sc_mine = F8 && wave * 64 < BM && wave * 64 < rows_u;
+  if constexpr (F8) {
+    const int R = row0 + min(min(wave, BM / 64 - 1) * 64 + lane, rows - 1);
+    sp += (int64_t)(p.a_rows ? p.a_rows[R] : R) * p.lds_a;
+  }
+  const int a_kshift = p.a_kshift, w_kshift = p.w_kshift;
+  const uint32_t cw = lds0 + wave * 1024;
+  auto copy_stage = [&](int s, int buf) {
+    const uint32_t d = __builtin_amdgcn_readfirstlane(cw + buf * STG);
+    const uint64_t b = reinterpret_cast<uint64_t>(wbase) + (uint64_t)(uint32_t)s * 128u;
+    const uint8_t* ws = reinterpret_cast<const uint8_t*>(
+        (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(b >> 32)) << 32 |
+        (uint32_t)__builtin_amdgcn_readfirstlane((int)b));
+#pragma unroll
+    for (int j = 0; j < WI; ++j) lds_copy16(ws, woff[j], d + j * 8192);
+#pragma unroll
+    for (int j = 0; j < XI; ++j)
+      if (j < nx) lds_copy16(xp[j] + (int64_t)s * 128, d + WB + j * 8192);
+    if (sc_mine) lds_copy4(sp + (s >> a_kshift), lds0 + buf * STG + WB + XB + wave * 256);
+  };
+  const int per_stage = WI + nx + (sc_mine ? 1 : 0);
+
+  const int KS = F8 ? p.K / 128 : p.K / 64;
+  const int rl = lane & 31, kh = lane >> 5;
+  // the weight scale of this wavefront's rows, tile layout (block i's rows lie
+  // in one 128-row tile). Read through the constant address space, as scalar
+  // loads: a vector load's wait would drain the copies in flight.
+  typedef const float __attribute__((address_space(4))) CFloat;
+  CFloat* wsp[NI];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+    wsp[i] = (CFloat*)(uintptr_t)(static_cast<const float*>(p.w_scale) +
+                                  (F8 && !WPC ? (int64_t)g * p.ws_gstride +
+                                                    (int64_t)(__builtin_amdgcn_readfirstlane(wrow_global(wrow(i))) / 128) *
+                                                        p.ldws
+                                              : 0));
+
+  f32x16 acc[NI][MJ];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < MJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+  // The K pipeline over the wavefront's first MJE token blocks (those with a
+  // token); the accumulators of the others keep their zeros.
+  auto pipeline = [&](auto mje_c) {
+    constexpr int MJE = decltype(mje_c)::value;
+#pragma unroll
+    for (int r = 0; r < (F8 ? RING - 1 : RING); ++r)
+      if (r < KS) copy_stage(r, r);
+    // Per stage: its first operands are in registers (read during the last
+    // MFMAs of the stage before). All but the last MFMA step run while the
+    // next step's operands are read; then the next stage's copies have landed
+    // (the one after's stay in flight with three buffers) -> barrier: they
+    // have landed everywhere, and everybody holds this stage's last operands,
+    // so that its buffer takes the copies of stage s + RING -> the last step,
+    // while the next stage's first operands are read.
+    auto landed = [&](int ahead) {
+      if (ahead && RING == 3) t8_wait(per_stage * ahead);
+      else wait_copies_upto<0>();
+    };
+    auto chunk = [&](const uint8_t* base, int row, int c) {
+      return *reinterpret_cast<const uint4*>(base + (row + rl) * 128 + ((c ^ t8_swz(rl)) * 16));
+    };
+    landed(0);
+    stage_barrier();
+    int buf = 0;
+    if constexpr (F8) {
+      auto frag = [&](const uint8_t* base, int row, int t) {
+        const uint4 a = chunk(base, row, 4 * t + 2 * kh), b = chunk(base, row, 4 * t + 2 * kh + 1);
+        i32x8 r;
+        r[0] = a.x; r[1] = a.y; r[2] = a.z; r[3] = a.w;
+        r[4] = b.x; r[5] = b.y; r[6] = b.z; r[7] = b.w;
+        return r;
+      };
+      // (a second set of weight operands, read ahead, would not fit the 256
+      // VGPRs: the stage's operands are read behind its barrier)
+      for (int s = 0; s < KS; ++s) {
+        if (s > 0) {
+          landed(RING == 3 && s + 1 < KS ? 1 : 0);
+          stage_barrier();
+        }
+        // (after the first operand reads, which the first MFMAs wait for)
+        auto refill = [&]() {
+          if (s + RING - 1 < KS) copy_stage(s + RING - 1, buf == 0 ? RING - 1 : buf - 1);
+        };
+        if constexpr (MJE == 0) refill();
+        if constexpr (MJE > 0) {
+          const uint8_t* sW = smem + buf * STG;
+          const uint8_t* sX = sW + WB;
+          const float* sS = reinterpret_cast<const float*>(sX + XB);
+          i32x8 wf[NI][2];
+          float sw[NI];
+#pragma unroll
+          for (int i = 0; i < NI; ++i) {
+            wf[i][0] = frag(sW, wrow(i), 0);
+            wf[i][1] = frag(sW, wrow(i), 1);
+            sw[i] = WPC ? 1.0f : wsp[i][s >> w_kshift];
+          }
+          // block pair n's MFMAs, then the scaling of pair n - 1
+          f32x16 tmp[2];
+          float sc[2];
+          i32x8 xf[2];
+          xf[0] = frag(sX, wm * 32, 0);
+          xf[1] = frag(sX, wm * 32, 1);
+          refill();
+#pragma unroll
+          for (int n = 0; n <= NI * MJE; ++n) {
+            if (n < NI * MJE) {
+              const int i = n % NI, j = n / NI, row = (2 * j + wm) * 32;
+              if (i == 0 && j > 0) {
+                xf[0] = frag(sX, row, 0);
+                xf[1] = frag(sX, row, 1);
+              }
+              sc[n & 1] = sS[row + rl] * sw[i];
+              tmp[n & 1] =
+                  __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wf[i][0], xf[0], f32x16{}, 0, 0, 0, 127, 0, 127);
+              tmp[n & 1] =
+                  __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wf[i][1], xf[1], tmp[n & 1], 0, 0, 0, 127, 0, 127);
+            }
+            if (n > 0) {
+              const int i = (n - 1) % NI, j = (n - 1) / NI;
+#pragma unroll
+              for (int r = 0; r < 16; ++r) acc[i][j][r] += tmp[(n - 1) & 1][r] * sc[(n - 1) & 1];
+            }
+          }
+        }
+        buf = buf == RING - 1 ? 0 : buf + 1;
+      }
+    } else {
+      union B8 {
+        uint4 u;
+        bf16x8 v;
+      };
+      constexpr int MR = MJE > 0 ? MJE : 1;
+      B8 wf[2][NI], xf[2][MR];
+      auto read_q = [&](int b, int q) {
+        const uint8_t* sW = smem + b * STG;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) wf[q & 1][i].u = chunk(sW, wrow(i), 2 * q + kh);
+#pragma unroll
+        for (int j = 0; j < MJE; ++j) xf[q & 1][j].u = chunk(sW + WB, (2 * j + wm) * 32, 2 * q + kh);
+      };
+      auto mma = [&](int q) {
+#pragma unroll
+        for (int i = 0; i < NI; ++i)
+#pragma unroll
+          for (int j = 0; j < MJE; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf[q & 1][i].v, xf[q & 1][j].v, acc[i][j], 0, 0, 0);
+      };
+      if constexpr (MJE > 0) read_q(0, 0);
+      for (int s = 0; s < KS; ++s) {
+        const int nb = buf == RING - 1 ? 0 : buf + 1;
+        if constexpr (MJE > 0) {
+#pragma unroll
+          for (int q = 0; q < 3; ++q) {
+            read_q(buf, q + 1);
+            mma(q);
+          }
+        }
+        if (s + 1 < KS) landed(s + 2 < KS ? 1 : 0);
+        stage_barrier();
+        if (s + RING < KS) copy_stage(s + RING, buf);
+        asm volatile("" ::: "memory");
+        if constexpr (MJE > 0) {
+          if (s + 1 < KS) read_q(nb, 0);
+          mma(3);
+        }
+        buf = nb;
+      }
+    }
+  };
+  // token blocks 2 j + wm with a token
+  const int mje = max(0, (cdiv(rows_u, 32) - wm + 1) / 2);
+  if constexpr (MJ == 4) {
+    if (mje == 0) pipeline(std::integral_constant<int, 0>{});
+    else if (mje == 1) pipeline(std::integral_constant<int, 1>{});
+    else if (mje == 2) pipeline(std::integral_constant<int, 2>{});
+    else if (mje == 3) pipeline(std::integral_constant<int, 3>{});
+    else pipeline(std::integral_constant<int, 4>{});
+  } else {
+    if (mje == 0) pipeline(std::integral_constant<int, 0>{});
+    else if (mje == 1) pipeline(std::integral_constant<int, 1>{});
+    else pipeline(std::integral_constant<int, 2>{});
+  }
+
+  // ---- epilogue: 64 tokens at a time, f32 sums in LDS ([64 tokens][256 tile
+  // rows], row n of token t at n ^ 4 (t % 16)), then 8 output channels of a
+  // token per thread
+  __syncthreads();  // every wavefront is done with the stage buffers
+  float* reg = reinterpret_cast<float*>(smem);
+  float* s_rw = reg + 64 * BN;
+  float *s_bs = s_rw + BM, *s_ws = s_bs + BN;
+  int* s_yr = reinterpret_cast<int*>(s_ws + BN);
+  static_assert((64 * BN + 2 * BM + 2 * BN) * 4 <= RING * STG, "epilogue regions");
+  if (tid < BM) {
+    s_rw[tid] = e_rw;
+    s_yr[tid] = e_yr;
+  }
+  if (tid < BN) {
+    s_bs[tid] = e_bs;
+    s_ws[tid] = e_ws;
+  }
+  const bool vec_ok = ((p.ldy & 7) == 0) && ((reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
+  const bool has_bias = p.bias != nullptr;
+#pragma unroll
+  for (int j = 0; j < MJ; ++j) {
+    if (j * 64 >= rows_u) break;
+    if (j) __syncthreads();  // the previous tokens have been read
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int n = wrow(i) + q * 8 + kh * 4;  // tile row of the register quad
+        *reinterpret_cast<float4*>(reg + (wm * 32 + rl) * BN + (n ^ (4 * (rl & 15)))) =
+            make_float4(acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]);
+      }
+    __syncthreads();
+    auto quad = [&](int t, int n) {
+      return *reinterpret_cast<const float4*>(reg + t * BN + (n ^ (4 * (t & 15))));
+    };
+    for (int e = tid; e < 64 * (BNO / 8); e += kT8Threads) {
+      const int t = e / (BNO / 8), c = (e % (BNO / 8)) * 8;  // token of the 64, first tile channel
+      const int tr = j * 64 + t;
+      if (tr >= rows || n0 + c >= nlim) continue;
+      const float4 g0 = quad(t, c), g1 = quad(t, c + 4);
+      const float vg[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+      float vu[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      if (ACT) {
+        const float4 h0 = quad(t, BN / 2 + c), h1 = quad(t, BN / 2 + c + 4);
+        vu[0] = h0.x; vu[1] = h0.y; vu[2] = h0.z; vu[3] = h0.w;
+        vu[4] = h1.x; vu[5] = h1.y; vu[6] = h1.z; vu[7] = h1.w;
+      }
+      const float rwt = s_rw[tr];
+      uint32_t packed[4];
+#pragma unroll
+      for (int k = 0; k < 8; k += 2) {
+        float o2[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          float v = vg[k + h];
+          if constexpr (F8 && WPC) v = v * s_ws[c + k + h];
+          if (has_bias) v += s_bs[c + k + h];
+          if (ACT) {
+            float u = vu[k + h];
+            if constexpr (F8 && WPC) u = u * s_ws[BN / 2 + c + k + h];
+            if (has_bias) u += s_bs[BN / 2 + c + k + h];
+            v = qmoe_act(p.act, v, u, p.act_p0, p.act_p1);
+          }
+          o2[h] = v * rwt;
+        }
+        packed[k / 2] = (uint32_t)f32_to_bf16(o2[0]) | ((uint32_t)f32_to_bf16(o2[1]) << 16);
+      }
+      uint16_t* dst = p.y + (int64_t)s_yr[tr] * p.ldy + n0 + c;
+      if (vec_ok && n0 + c + 8 <= nlim) {
+        *reinterpret_cast<uint4*>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+      } else {
+        for (int k = 0; k < 8 && n0 + c + k < nlim; ++k) dst[k] = (uint16_t)(packed[k / 2] >> ((k & 1) * 16));
+      }
+    }
+  }
+}
+
+template <bool F8, int BM, bool ACT, bool WPC>
+void t8_launch_shape(const GemmParams& p, hipStream_t st) {
+  const int n_tiles = cdiv(ACT ? p.N / 2 : p.N, ACT ? kT8BN / 2 : kT8BN);
+  const int m_tiles = p.group_offs ? cdiv(cdiv(p.M, BM) + std::min(p.slots, p.M), kXcds) * kXcds : cdiv(p.M, BM);
+  const int grid = p.group_offs ? m_tiles * n_tiles : cdiv(m_tiles * n_tiles, kXcds) * kXcds;
+  hipLaunchKernelGGL((t8_gemm_kernel<F8, BM, ACT, WPC>), dim3(grid), dim3(kT8Threads), 0, st, p, m_tiles, n_tiles);
+}
+
+template <bool WPC>
+void t8_launch_f8(const GemmParams& p, int bm, hipStream_t st) {
+  const bool act = p.act != QA_NONE;
+  if (bm == 256) act ? t8_launch_shape<true, 256, true, WPC>(p, st) : t8_launch_shape<true, 256, false, WPC>(p, st);
+  else act ? t8_launch_shape<true, 128, true, WPC>(p, st) : t8_launch_shape<true, 128, false, WPC>(p, st);
+}
+
+}  // namespace
+
+// Token-tile height of the problem on this kernel, 0 when another one takes
+// it. `f8`: block-scaled e4m3 codes (else bf16 on both sides).
+int qmoe_t8_plan(const GemmParams& p, bool f8) {
+  if (p.M <= 0 || p.N <= 0 || p.K <= 0 || (p.K % (f8 ? 128 : 64)) != 0) return 0;
+  if (p.act != QA_NONE && (p.N % 2) != 0) return 0;
+  const bool wpc = p.w_kshift >= 31;
+  if (f8 && (p.wfmt != 0 || (!wpc && (p.ws_bn != 128 || (p.act != QA_NONE && ((p.N / 2) % 128) != 0))))) return 0;
+  if (((p.lda * (f8 ? 1 : 2)) % 16) != 0 || (p.ldw % 16) != 0 || (p.w_gstride % 16) != 0) return 0;
+  if ((reinterpret_cast<uintptr_t>(p.a) & 15) || (reinterpret_cast<uintptr_t>(p.w) & 15)) return 0;
+  if ((int64_t)p.ldw * p.N >= ((int64_t)1 << 32)) return 0;
+  // bf16: dense linears (the grouped bf16 layers keep the generic tiles)
+  if (!f8 && (p.group_offs || p.act != QA_NONE)) return 0;
+  const char* env = getenv("QMOE_T8_BM");  // tuning knob: 128, 256 or 0 (off)
+  if (env) return atoi(env) == 128 || atoi(env) == 256 ? atoi(env) : 0;
+  if (p.group_offs) {
+    // measured on MI355X (DeepSeek-V3 routed experts, 256 experts, top 8,
+    // per-channel weights; gemm_f8.hip's tiles, 128-, 256-token tiles): 64
+    // tokens 1041 / 1029 / 1025 us, 256 tokens 1414 / 1343 / 1503, 2048
+    // 2659 / 2356 / 2558, 8192 (128 x 128 tiles) 5989 / 5591 / 5162
+    return p.M / std::max(1, std::min(p.slots, p.M)) > 192 ? 256 : 128;
+  }
+  // Dense: the tile height with the cheaper rounds over the 256 CUs (a round of
+  // 256-token tiles takes 1.57 to 1.73 times one of 128-token tiles: K 7168, N
+  // 18432, 512 / 1024 / 4096 / 8192 tokens 142 / 211 / 735 / 1469 us in
+  // 128-token tiles, 119 / 236 / 642 / 1246 in 256-token tiles), if it has
+  // work for more than half of them; else the smaller tiles and K splits of
+  // the other kernels (K 4096, N 4096, 1024 tokens, 128 tiles: 50 us here,
+  // 41 there; K 2048, N 7168, 1000 tokens, 224 tiles: 32 and 42).
+  const int n_tiles = cdiv(p.act != QA_NONE ? p.N / 2 : p.N, p.act != QA_NONE ? kT8BN / 2 : kT8BN);
+  const int64_t t128 = (int64_t)cdiv(p.M, 128) * n_tiles, t256 = (int64_t)cdiv(p.M, 256) * n_tiles;
+  const int bm = cdiv<int64_t>(t128, 256) * 100 <= cdiv<int64_t>(t256, 256) * 168 ? 128 : 256;
+  return (bm == 128 ? t128 : t256) >= 140 ? bm : 0;
+}
+
+int qmoe_t8_launch(GemmParams p, bool f8, hipStream_t st) {
+  const int bm = qmoe_t8_plan(p, f8);
+  if (!bm) return QMOE_ERR_ARG;
+  p.ksplit = 1;
+  if (!f8) bm == 256 ? t8_launch_shape<false, 256, false, false>(p, st) : t8_launch_shape<false, 128, false, false>(p, st);
+  else if (p.w_kshift >= 31) t8_launch_f8<true>(p, bm, st);
+  else t8_launch_f8<false>(p, bm, st);
+  return hipGetLastError() == hipSuccess ? QMOE_OK : QMOE_ERR_LAUNCH;
+}

@@ -62,6 +62,26 @@ __device__ __forceinline__ void wait_copies_upto() {
   __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (7 << 4) | (15 << 8));
 }
 
+// One direct global -> LDS copy of 16 bytes per lane: `lds` (byte address,
+// wave-uniform) + 16 * lane <- src. Written as assembly so that the compiler
+// does not order it against the LDS reads: it would drain every copy in
+// flight before a read of a ring buffer whose index it cannot resolve. The
+// kernel's own counted waits and barriers order them. The instruction has no
+// register result and takes its address registers when it issues; the
+// s_nop is the wait state between a write of M0 and its use. A kernel that
+// uses these makes no other use of M0 (no copy builtins beside them).
+__device__ __forceinline__ void lds_copy16(const uint8_t* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+}
+__device__ __forceinline__ void lds_copy16(const uint8_t* base, uint32_t off, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
+               : "memory");
+}
+// The same for 4 bytes per lane (`lds` + 4 * lane).
+__device__ __forceinline__ void lds_copy4(const void* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(src) : "memory");
+}
+
 template <int BM>
 __device__ __forceinline__ bool tile_group(const GemmParams& p, int y, int& g, int& row0, int& rows,
                                               int* s_info) {

@@ -80,21 +80,6 @@ __device__ __forceinline__ bf16x8 as_bf16x8_u4(const uint4& x) {
   return c.v;
 }
 
-// One direct global -> LDS copy of 16 bytes per lane: `lds` (byte address,
-// wave-uniform) + 16 * lane <- src. Written as assembly so that the compiler
-// does not order it against the LDS reads: it would drain every copy in
-// flight before a read of a ring buffer whose index it cannot resolve. The
-// kernel's own counted waits and barriers order them. The instruction has no
-// register result and takes its address registers when it issues; the
-// s_nop is the wait state between a write of M0 and its use.
-__device__ __forceinline__ void w4_copy16(const uint8_t* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
-}
-__device__ __forceinline__ void w4_copy16(const uint8_t* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
-               : "memory", "m0");
-}
-
 // FMT: 0 MXFP4, 1 NVFP4, 2 INT4
 template <int BM, int KG, bool ACT, int FMT>
 __global__ __launch_bounds__(KG * kThreads, 2) void w4_gemm_kernel(const GemmParams p, int m_tiles, int n_tiles) {
@@ -209,7 +194,7 @@ __global__ __launch_bounds__(KG * kThreads, 2) void w4_gemm_kernel(const GemmPar
     const uint32_t b0 = (uint32_t)min(max(b + wc16, 0), rowb - 16);
     const uint32_t b1 = (uint32_t)min(max(b + (wc16 ^ 16), 0), rowb - 16);
 #pragma unroll
-    for (int j = 0; j < WI; ++j) w4_copy16(wbase, roff[j] + (j & 1 ? b1 : b0), wdst + j * 1024);
+    for (int j = 0; j < WI; ++j) lds_copy16(wbase, roff[j] + (j & 1 ? b1 : b0), wdst + j * 1024);
   };
 
   // ---- weight scales: lane (row l % 32, half h) of weight block i needs, for
@@ -274,7 +259,7 @@ __global__ __launch_bounds__(KG * kThreads, 2) void w4_gemm_kernel(const GemmPar
       for (int h = 0; h < PB; ++h)
 #pragma unroll
         for (int j = 0; j < MJE; ++j)
-          w4_copy16(xp[j] + min(ks + h, KS - 1) * 128, xdst + buf * AB + h * SB + j * 4096);
+          lds_copy16(xp[j] + min(ks + h, KS - 1) * 128, xdst + buf * AB + h * SB + j * 4096);
     };
     uint4 wc[4][NI];  // codes of a line's four stages
     auto read_line = [&]() {
