@@ -130,3 +130,39 @@ def test_bf16(monkeypatch, bm, M, N, K):
         got = ops.gemm(_capi.W16A16, x, w, bias=bias)
     assert plans[0][4] == "tiled_8w"
     _check(got, x.double() @ w.double().t() + bias.double(), x.double().abs() @ w.double().abs().t() + bias.double().abs())
+
+
+@pytest.mark.parametrize("kind", ["fp8", "bf16"])
+@pytest.mark.parametrize("M,N", [(1024, 18432), (2047, 18432), (1500, 14300), (769, 18300)])
+def test_dense_rounds_of_two_heights(monkeypatch, kind, M, N):
+    """Problems whose last, partly filled round of 256-token tiles runs as
+    128-token tiles (the last of the four: all in one height): the same sums
+    in the same order as 128-token tiles throughout."""
+    from qmoe import _capi, ops
+
+    g = _gen(M + N)
+    K = 256
+    rw = torch.rand(M, device="cuda", generator=g).to(torch.bfloat16)
+    perm = torch.randperm(M, generator=torch.Generator().manual_seed(3)).to(dtype=torch.int32, device="cuda")
+    if kind == "fp8":
+        N = (N + 127) // 128 * 128
+        x, w = _codes((M, K), g), _codes((N, K), g)
+        xs, ws = _scales((M, K // 128), g), _scales((N // 128, K // 128), g)
+        call = lambda **kw: ops.gemm(_capi.W8A8_BLK, x.view(torch.uint8), w.view(torch.uint8), a_scale=xs,  # noqa: E731
+                                     w_scale=ws, ws_bn=128, **kw)
+        xd = x.double() * xs.double().repeat_interleave(128, 1)
+        wd = w.double() * ws.double().repeat_interleave(128, 0).repeat_interleave(128, 1)
+    else:
+        x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
+        w = torch.randn((N, K), device="cuda", generator=g).to(torch.bfloat16)
+        call = lambda **kw: ops.gemm(_capi.W16A16, x, w, **kw)  # noqa: E731
+        xd, wd = x.double(), w.double()
+    for kw in ({}, dict(row_weight=rw, y_rows=perm)):
+        monkeypatch.delenv("QMOE_T8_BM", raising=False)
+        with ops.record_plans() as plans:
+            got = call(**kw)
+        assert plans[0][4] == "tiled_8w"
+        monkeypatch.setenv("QMOE_T8_BM", "128")
+        assert torch.equal(got, call(**kw))
+        if not kw:
+            _check(got, xd @ wd.t(), xd.abs() @ wd.abs().t())

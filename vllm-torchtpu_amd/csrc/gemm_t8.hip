@@ -413,9 +413,61 @@ void t8_launch_f8(const GemmParams& p, int bm, hipStream_t st) {
   else act ? t8_launch_shape<true, 128, true, WPC>(p, st) : t8_launch_shape<true, 128, false, WPC>(p, st);
 }
 
+// Dense: how many 256-token tiles (of every weight tile) come first; the rows
+// after them run as 128-token tiles in a second launch. The candidates are
+// 128-token tiles alone, 256-token tiles alone, and whole rounds of 256-token
+// tiles over the 256 CUs with the last round, or the last two, as 128-token
+// tiles. A round of 256-token tiles takes 1.57 to 1.73 times one of 128-token
+// tiles (K 7168, N 18432, 512 / 1024 / 4096 / 8192 tokens 142 / 211 / 735 /
+// 1469 us in 128-token tiles, 119 / 236 / 642 / 1246 in 256-token tiles).
+// Measured, two heights / 128 / 256 alone: e4m3 K 7168, N 18432 at 1024 / 2048
+// tokens 197 / 205 / 227, 311 / 341 / 347 us; K 4096, N 6144 at 3000 116 / 125
+// / 141; bf16 K 7168, N 18432 at 1024 296 / 325 / 364, K 4096, N 6144 at 3000
+// 171 / 185 / 209.
+int t8_tall_tiles(int M, int n_tiles) {
+  const int64_t m256 = cdiv(M, 256), rounds = cdiv<int64_t>(m256 * n_tiles, 256);
+  int64_t best = 0, best_cost = -1;
+  auto consider = [&](int64_t tall) {
+    const int64_t rest = std::max<int64_t>(M - tall * 256, 0);
+    int64_t cost = cdiv<int64_t>(tall * n_tiles, 256) * 168 + cdiv<int64_t>(cdiv<int64_t>(rest, 128) * n_tiles, 256) * 100;
+    if (tall > 0 && rest > 0) cost += 10;  // the second launch
+    if (best_cost < 0 || cost < best_cost) best = tall, best_cost = cost;
+  };
+  consider(0);
+  consider(m256);
+  for (int64_t r = rounds - 1; r > 0 && r >= rounds - 2; --r) consider(r * 256 / n_tiles);
+  return (int)best;
+}
+
+// The rows from `row` on of a dense problem
+GemmParams t8_rows_from(GemmParams p, int row, int a_bytes) {
+  p.M -= row;
+  if (p.a_rows) {
+    p.a_rows += row;
+  } else {
+    p.a = static_cast<const uint8_t*>(p.a) + (int64_t)row * p.lda * a_bytes;
+    if (p.a_scale) p.a_scale += (int64_t)row * p.lds_a;
+  }
+  if (p.row_weight) p.row_weight += row;
+  if (p.y_rows) p.y_rows += row;
+  else p.y += (int64_t)row * p.ldy;
+  return p;
+}
+
+void t8_launch(const GemmParams& p, bool f8, int bm, hipStream_t st) {
+  if (!f8) bm == 256 ? t8_launch_shape<false, 256, false, false>(p, st) : t8_launch_shape<false, 128, false, false>(p, st);
+  else if (p.w_kshift >= 31) t8_launch_f8<true>(p, bm, st);
+  else t8_launch_f8<false>(p, bm, st);
+}
+
+int t8_n_tiles(const GemmParams& p) {
+  return cdiv(p.act != QA_NONE ? p.N / 2 : p.N, p.act != QA_NONE ? kT8BN / 2 : kT8BN);
+}
+
 }  // namespace
 
-// Token-tile height of the problem on this kernel, 0 when another one takes
+// Token-tile height of the problem on this kernel (256 also where the last
+// rows of a dense problem run as 128-token tiles), 0 when another one takes
 // it. `f8`: block-scaled e4m3 codes (else bf16 on both sides).
 int qmoe_t8_plan(const GemmParams& p, bool f8) {
   if (p.M <= 0 || p.N <= 0 || p.K <= 0 || (p.K % (f8 ? 128 : 64)) != 0) return 0;
@@ -436,25 +488,28 @@ int qmoe_t8_plan(const GemmParams& p, bool f8) {
     // 2659 / 2356 / 2558, 8192 (128 x 128 tiles) 5989 / 5591 / 5162
     return p.M / std::max(1, std::min(p.slots, p.M)) > 192 ? 256 : 128;
   }
-  // Dense: the tile height with the cheaper rounds over the 256 CUs (a round of
-  // 256-token tiles takes 1.57 to 1.73 times one of 128-token tiles: K 7168, N
-  // 18432, 512 / 1024 / 4096 / 8192 tokens 142 / 211 / 735 / 1469 us in
-  // 128-token tiles, 119 / 236 / 642 / 1246 in 256-token tiles), if it has
-  // work for more than half of them; else the smaller tiles and K splits of
-  // the other kernels (K 4096, N 4096, 1024 tokens, 128 tiles: 50 us here,
-  // 41 there; K 2048, N 7168, 1000 tokens, 224 tiles: 32 and 42).
-  const int n_tiles = cdiv(p.act != QA_NONE ? p.N / 2 : p.N, p.act != QA_NONE ? kT8BN / 2 : kT8BN);
-  const int64_t t128 = (int64_t)cdiv(p.M, 128) * n_tiles, t256 = (int64_t)cdiv(p.M, 256) * n_tiles;
-  const int bm = cdiv<int64_t>(t128, 256) * 100 <= cdiv<int64_t>(t256, 256) * 168 ? 128 : 256;
-  return (bm == 128 ? t128 : t256) >= 140 ? bm : 0;
+  // Dense, if it has work for more than half of the CUs; else the smaller
+  // tiles and K splits of the other kernels (K 4096, N 4096, 1024 tokens, 128
+  // tiles: 50 us here, 41 there; K 2048, N 7168, 1000 tokens, 224 tiles: 32
+  // and 42).
+  const int n_tiles = t8_n_tiles(p), tall = t8_tall_tiles(p.M, n_tiles);
+  const int64_t tiles = (int64_t)(tall + cdiv(std::max(p.M - (int64_t)tall * 256, (int64_t)0), (int64_t)128)) * n_tiles;
+  return tiles >= 140 ? (tall ? 256 : 128) : 0;
 }
 
 int qmoe_t8_launch(GemmParams p, bool f8, hipStream_t st) {
   const int bm = qmoe_t8_plan(p, f8);
   if (!bm) return QMOE_ERR_ARG;
   p.ksplit = 1;
-  if (!f8) bm == 256 ? t8_launch_shape<false, 256, false, false>(p, st) : t8_launch_shape<false, 128, false, false>(p, st);
-  else if (p.w_kshift >= 31) t8_launch_f8<true>(p, bm, st);
-  else t8_launch_f8<false>(p, bm, st);
+  const bool forced = getenv("QMOE_T8_BM") != nullptr;
+  const int tall = bm == 256 && !p.group_offs && !forced ? t8_tall_tiles(p.M, t8_n_tiles(p)) : 0;
+  if (tall > 0 && (int64_t)tall * 256 < p.M) {
+    GemmParams top = p;
+    top.M = tall * 256;
+    t8_launch(top, f8, 256, st);
+    t8_launch(t8_rows_from(p, tall * 256, f8 ? 1 : 2), f8, 128, st);
+  } else {
+    t8_launch(p, f8, bm, st);
+  }
   return hipGetLastError() == hipSuccess ? QMOE_OK : QMOE_ERR_LAUNCH;
 }
