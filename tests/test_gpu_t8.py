@@ -57,7 +57,8 @@ def test_dense_tiles(monkeypatch, bm, M, N, K):
 
 @pytest.mark.parametrize("bm", ["128", "256"])
 @pytest.mark.parametrize("recipe,N,K,act", [("tiles", 512, 384, "silu"), ("tiles", 384, 256, None),
-                                            ("channel", 200, 640, None), ("channel", 1026, 512, "silu")])
+                                            ("channel", 200, 640, None), ("channel", 1026, 512, "silu"),
+                                            ("e5m2", 1026, 640, "silu"), ("e5m2", 512, 512, None)])
 def test_grouped(monkeypatch, bm, recipe, N, K, act):
     """Experts of 0 to 260 rows, gathered tokens, scattered rows, routing weights and bias."""
     from qmoe import _capi, ops
@@ -67,6 +68,8 @@ def test_grouped(monkeypatch, bm, recipe, N, K, act):
     E, M, T = len(counts), sum(counts), 150
     x, w = _codes((T, K), g), _codes((E, N, K), g)
     tiles = recipe == "tiles"
+    if recipe == "e5m2":
+        w = w.float().to(torch.float8_e5m2)
     nb = (K + 511) // 512
     xs = _scales((T, K // 128 if tiles else nb), g)
     ws = _scales((E, N // 128, K // 128) if tiles else (E, N), g)
@@ -81,7 +84,8 @@ def test_grouped(monkeypatch, bm, recipe, N, K, act):
         monkeypatch.setenv("QMOE_T8_BM", v)
         out = torch.empty((M, N // 2 if act else N), dtype=torch.bfloat16, device="cuda")
         return ops.gemm(_capi.W8A8_BLK if tiles else _capi.W8A8_GMM, x.view(torch.uint8), w.view(torch.uint8),
-                        a_scale=xs, w_scale=ws, ws_bn=128 if tiles else 1, bias=bias, group_offs=offs,
+                        a_scale=xs, w_scale=ws, ws_bn=128 if tiles else 1, wfmt=2 if recipe == "e5m2" else 0,
+                        bias=bias, group_offs=offs,
                         active=torch.arange(E, **i32), num_active=torch.tensor([E], **i32), slots=E, max_rows=T, M=M,
                         a_rows=rows, activation=act, row_weight=rw, y_rows=perm, out=out)
 

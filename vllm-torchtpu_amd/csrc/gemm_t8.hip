@@ -1,6 +1,6 @@
 // Tiles of eight wavefronts (one workgroup per CU, two wavefronts per SIMD):
-// block-scaled FP8 (QK_W8A8_BLK, e4m3 codes: 128 x 128 weight tiles or the
-// grouped matmul's per-channel weights, activation scales per 128 or 512
+// block-scaled FP8 (QK_W8A8_BLK: 128 x 128 tiles of e4m3 weights or the
+// grouped matmul's per-channel e4m3 or e5m2 weights, activation scales per 128 or 512
 // columns) and bf16 x bf16 (QK_W16A16), dense or grouped.
 //
 //  * What bounds it: the matrix cores with the vector ALU and the operand
@@ -50,9 +50,10 @@ __device__ __forceinline__ void t8_wait(int n) {
   }
 }
 
-// F8: block-scaled e4m3; else bf16. WPC (F8): one weight scale per weight row,
-// applied in the epilogue, instead of one per 128 x 128 tile.
-template <bool F8, int BM, bool ACT, bool WPC>
+// F8: block-scaled 1-byte floats; else bf16. WPC (F8): one weight scale per
+// weight row, applied in the epilogue, instead of one per 128 x 128 tile. WF:
+// weight format code of the MFMA, 0 e4m3, 1 e5m2 (activations are e4m3).
+template <bool F8, int BM, bool ACT, bool WPC, int WF>
 __global__ __launch_bounds__(kT8Threads, 2) void t8_gemm_kernel(const GemmParams p, int m_tiles, int n_tiles) {
   constexpr int BN = kT8BN, BNO = ACT ? BN / 2 : BN;
   constexpr int NI = 2, MJ = BM / 64;            // 32-row weight blocks, 32-token blocks per wavefront
@@ -251,9 +252,9 @@ __global__ __launch_bounds__(kT8Threads, 2) void t8_gemm_kernel(const GemmParams
               }
               sc[n & 1] = sS[row + rl] * sw[i];
               tmp[n & 1] =
-                  __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wf[i][0], xf[0], f32x16{}, 0, 0, 0, 127, 0, 127);
+                  __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wf[i][0], xf[0], f32x16{}, WF, 0, 0, 127, 0, 127);
               tmp[n & 1] =
-                  __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wf[i][1], xf[1], tmp[n & 1], 0, 0, 0, 127, 0, 127);
+                  __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wf[i][1], xf[1], tmp[n & 1], WF, 0, 0, 127, 0, 127);
             }
             if (n > 0) {
               const int i = (n - 1) % NI, j = (n - 1) / NI;
@@ -398,19 +399,19 @@ __global__ __launch_bounds__(kT8Threads, 2) void t8_gemm_kernel(const GemmParams
   }
 }
 
-template <bool F8, int BM, bool ACT, bool WPC>
+template <bool F8, int BM, bool ACT, bool WPC, int WF = 0>
 void t8_launch_shape(const GemmParams& p, hipStream_t st) {
   const int n_tiles = cdiv(ACT ? p.N / 2 : p.N, ACT ? kT8BN / 2 : kT8BN);
   const int m_tiles = p.group_offs ? cdiv(cdiv(p.M, BM) + std::min(p.slots, p.M), kXcds) * kXcds : cdiv(p.M, BM);
   const int grid = p.group_offs ? m_tiles * n_tiles : cdiv(m_tiles * n_tiles, kXcds) * kXcds;
-  hipLaunchKernelGGL((t8_gemm_kernel<F8, BM, ACT, WPC>), dim3(grid), dim3(kT8Threads), 0, st, p, m_tiles, n_tiles);
+  hipLaunchKernelGGL((t8_gemm_kernel<F8, BM, ACT, WPC, WF>), dim3(grid), dim3(kT8Threads), 0, st, p, m_tiles, n_tiles);
 }
 
-template <bool WPC>
+template <bool WPC, int WF = 0>
 void t8_launch_f8(const GemmParams& p, int bm, hipStream_t st) {
   const bool act = p.act != QA_NONE;
-  if (bm == 256) act ? t8_launch_shape<true, 256, true, WPC>(p, st) : t8_launch_shape<true, 256, false, WPC>(p, st);
-  else act ? t8_launch_shape<true, 128, true, WPC>(p, st) : t8_launch_shape<true, 128, false, WPC>(p, st);
+  if (bm == 256) act ? t8_launch_shape<true, 256, true, WPC, WF>(p, st) : t8_launch_shape<true, 256, false, WPC, WF>(p, st);
+  else act ? t8_launch_shape<true, 128, true, WPC, WF>(p, st) : t8_launch_shape<true, 128, false, WPC, WF>(p, st);
 }
 
 // Dense: how many 256-token tiles (of every weight tile) come first; the rows
@@ -456,7 +457,7 @@ GemmParams t8_rows_from(GemmParams p, int row, int a_bytes) {
 
 void t8_launch(const GemmParams& p, bool f8, int bm, hipStream_t st) {
   if (!f8) bm == 256 ? t8_launch_shape<false, 256, false, false>(p, st) : t8_launch_shape<false, 128, false, false>(p, st);
-  else if (p.w_kshift >= 31) t8_launch_f8<true>(p, bm, st);
+  else if (p.w_kshift >= 31) p.wfmt == 2 ? t8_launch_f8<true, 1>(p, bm, st) : t8_launch_f8<true>(p, bm, st);
   else t8_launch_f8<false>(p, bm, st);
 }
 
@@ -468,12 +469,12 @@ int t8_n_tiles(const GemmParams& p) {
 
 // Token-tile height of the problem on this kernel (256 also where the last
 // rows of a dense problem run as 128-token tiles), 0 when another one takes
-// it. `f8`: block-scaled e4m3 codes (else bf16 on both sides).
+// it. `f8`: block-scaled codes (else bf16 on both sides).
 int qmoe_t8_plan(const GemmParams& p, bool f8) {
   if (p.M <= 0 || p.N <= 0 || p.K <= 0 || (p.K % (f8 ? 128 : 64)) != 0) return 0;
   if (p.act != QA_NONE && (p.N % 2) != 0) return 0;
   const bool wpc = p.w_kshift >= 31;
-  if (f8 && (p.wfmt != 0 || (!wpc && (p.ws_bn != 128 || (p.act != QA_NONE && ((p.N / 2) % 128) != 0))))) return 0;
+  if (f8 && (p.wfmt == 1 || (p.wfmt != 0 && !wpc) || (!wpc && (p.ws_bn != 128 || (p.act != QA_NONE && ((p.N / 2) % 128) != 0))))) return 0;
   if (((p.lda * (f8 ? 1 : 2)) % 16) != 0 || (p.ldw % 16) != 0 || (p.w_gstride % 16) != 0) return 0;
   if ((reinterpret_cast<uintptr_t>(p.a) & 15) || (reinterpret_cast<uintptr_t>(p.w) & 15)) return 0;
   if ((int64_t)p.ldw * p.N >= ((int64_t)1 << 32)) return 0;
