@@ -111,3 +111,25 @@ def test_grouped(monkeypatch, fmt, bm, K, N, act):
                 h = (u + 1) * g * torch.sigmoid(1.702 * g)
         w = rw[r].double()[:, None]
         _check(out[perm[r].long()], h * w, mag * w)
+
+
+@pytest.mark.parametrize("K,ks", [(2496, None), (2560, None), (2624, "1"), (2624, "3"), (64, "1"), (384, None)])
+@pytest.mark.parametrize("M", [33, 129])
+def test_ring_fused_activation(monkeypatch, K, ks, M):
+    """The NVFP4 ring below and above the K from which two K groups share a
+    workgroup, halves of equal and unequal stages, gate and up rows."""
+    from qmoe import ops
+
+    I = 257
+    gen = torch.Generator(device="cuda").manual_seed(K + M)
+    codes, s, val = _weights("nv", 2 * I, K, 0, gen)
+    x = torch.randn((M, K), device="cuda", generator=gen).to(torch.bfloat16)
+    monkeypatch.setenv("QMOE_SKINNY_MAX_ROWS", "0")
+    monkeypatch.setenv("QMOE_SKINNY_ROW_SPLIT", "0")
+    if ks:
+        monkeypatch.setenv("QMOE_W4_KSPLIT", ks)
+    got = ops.gemm(_kind("nv"), x, codes, w_scale=s, activation="silu")
+    h, mag = x.double() @ val.t(), x.double().abs() @ val.abs().t()
+    g, u = h[:, :I], h[:, I:]
+    mag = 2 * ((u.abs() + 1) * mag[:, :I] + (g.abs() + 1) * mag[:, I:]) + 1
+    _check(got, g * torch.sigmoid(g) * u, mag)

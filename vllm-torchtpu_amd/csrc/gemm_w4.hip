@@ -55,6 +55,7 @@ namespace {
 
 using rsrc_t = __amdgpu_buffer_rsrc_t;
 constexpr int kW4BN = 256;  // weight rows per tile
+constexpr int kCusPerXcd = 32;
 
 __device__ __forceinline__ int w4_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
@@ -524,9 +525,13 @@ struct W4Shape {
 // four stages ahead, with the operand reads and copies of a stage spread
 // over its MFMAs. It spends fewer instructions per stage than the line
 // pipeline above, and with one workgroup per CU that is what counts: NVFP4 K
-// 2880, N 5760 at 128 / 203 tokens 23.4 / 28.1 us against 26.0 / 32.0.
-template <int BM, bool ACT, int FMT>
-__global__ __launch_bounds__(kThreads) void w4_ring_kernel(const GemmParams p, int m_tiles, int n_tiles) {
+// 2880, N 5760 at 128 / 203 tokens 22.6 / 27.7 us against 26.0 / 32.0. What
+// bounds it is the expansion, about 1500 cycles per stage on the vector ALU:
+// two K groups of four wavefronts (KG 2, their sums added through LDS) shorten
+// a long chain of stages by a few percent only (203 tokens 28.6 -> 27.7 us, K
+// 4096, N 4096 38.3 -> 33.1), the K split the rest (28.6).
+template <int BM, int KG, bool ACT, int FMT>
+__global__ __launch_bounds__(KG * kThreads) void w4_ring_kernel(const GemmParams p, int m_tiles, int n_tiles) {
   constexpr bool NV = FMT == 1, I4 = FMT == 2;
   using S = W4Shape<BM>;
   constexpr int BN = kW4BN;
@@ -534,13 +539,18 @@ __global__ __launch_bounds__(kThreads) void w4_ring_kernel(const GemmParams p, i
   constexpr int BNO = ACT ? BN / 2 : BN;  // output channels per tile
   static_assert(!ACT || NI % 2 == 0, "fused activation pairs gate and up blocks");
 
-  // four LDS stages of 64 k: activations [BM][128 B], codes [BN][32 B]
-  __shared__ __align__(1024) uint8_t sA0[BM * 128], sA1[BM * 128], sA2[BM * 128], sA3[BM * 128];
-  __shared__ __align__(1024) uint8_t sW0[BN * 32], sW1[BN * 32], sW2[BN * 32], sW3[BN * 32];
+  // four LDS stages of 64 k per K group: activations [BM][128 B], codes [BN][32 B]
+  constexpr int AB = BM * 128, WB = BN * 32;
+  __shared__ __align__(1024) uint8_t sA0s[KG * AB], sA1s[KG * AB], sA2s[KG * AB], sA3s[KG * AB];
+  __shared__ __align__(1024) uint8_t sW0s[KG * WB], sW1s[KG * WB], sW2s[KG * WB], sW3s[KG * WB];
   __shared__ float s_sx[BM], s_rw[BM], s_ws[BN], s_bs[BN];
   __shared__ int s_yr[BM];
 
-  const int tid = threadIdx.x;
+  // K group of the wavefront; threads and wavefronts count within the group
+  const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kThreads) : 0;
+  const int tid = KG > 1 ? (int)threadIdx.x % kThreads : (int)threadIdx.x;
+  uint8_t *sA0 = sA0s + kg * AB, *sA1 = sA1s + kg * AB, *sA2 = sA2s + kg * AB, *sA3 = sA3s + kg * AB;
+  uint8_t *sW0 = sW0s + kg * WB, *sW1 = sW1s + kg * WB, *sW2 = sW2s + kg * WB, *sW3 = sW3s + kg * WB;
   const int lane = tid & 63, wave = tid >> 6;
   const int wn = wave % S::WN, wm = wave / S::WN;
 
@@ -604,11 +614,14 @@ __global__ __launch_bounds__(kThreads) void w4_ring_kernel(const GemmParams p, i
     woff[j] = (uint32_t)wrow_global(r) * (uint32_t)p.ldw + (lane & 1) * 16;
   }
 
-  // split-K: this workgroup's K range in 64-k stages
+  // split-K: this workgroup's K range in 64-k stages, dealt to the K groups
+  // (the first may have one stage more: `most`, the others at least `least`)
   const int NU = p.K / 64;
-  const int u0 = (int)((int64_t)NU * blockIdx.z / p.ksplit);
+  const int wg0 = (int)((int64_t)NU * blockIdx.z / p.ksplit);
   const int u1 = (int)((int64_t)NU * (blockIdx.z + 1) / p.ksplit);
-  const int KS = u1 - u0;
+  const int most = cdiv(u1 - wg0, KG), least = (u1 - wg0) / KG;
+  const int u0 = wg0 + kg * most;
+  const int KS = kg == 0 ? most : least;
   const int rl = lane & 31, kh = lane >> 5;
   auto wrow = [&](int i) { return tile_wrow<BN, TN, NI, ACT>(wn, i); };
   uint32_t eoff[NI];
@@ -618,7 +631,8 @@ __global__ __launch_bounds__(kThreads) void w4_ring_kernel(const GemmParams p, i
   const int lg = I4 ? (p.wq_group == 32 ? 5 : (p.wq_group == 64 ? 6 : 7)) : 0;  // log2(group)
   uint32_t we[4][NI];  // scales of the stages in flight (stage s in set s % 4)
   auto copy_stage = [&](uint8_t* dA, uint8_t* dW, int e, int ks) {
-    const uint32_t st = (uint32_t)(u0 + ks);
+    // (a group without stages fetches one that it never uses)
+    const uint32_t st = (uint32_t)(KG > 1 ? min(u0 + max(ks, 0), NU - 1) : u0 + ks);
 #pragma unroll
     for (int j = 0; j < WI; ++j) {
       uint32_t o = woff[j];
@@ -723,11 +737,12 @@ __global__ __launch_bounds__(kThreads) void w4_ring_kernel(const GemmParams p, i
 #pragma unroll
       for (int i = 0; i < NI; ++i) eb[i] = we[e][i];
       copy_stage(fA, fW, e, min(s + 4, KS - 1));
+      if (KG > 1 && s >= KS) return;  // the other group's last stage
       mma_stage(t, eb);
       read_stage(nA, nW, t ^ 1);
       interleave<0, NM, NR, CPS>();
     };
-    if (KS > 0) {
+    if (most > 0) {
       copy_stage(sA0, sW0, 0, 0);
       copy_stage(sA1, sW1, 1, min(1, KS - 1));
       copy_stage(sA2, sW2, 2, min(2, KS - 1));
@@ -736,15 +751,16 @@ __global__ __launch_bounds__(kThreads) void w4_ring_kernel(const GemmParams p, i
       __syncthreads();
       read_stage(sA0, sW0, 0);
       int s = 0;
-      for (; s + 4 <= KS; s += 4) {
+      for (; s + 4 <= least; s += 4) {
         stage(sA0, sW0, sA1, sW1, 0, s, 0);
         stage(sA1, sW1, sA2, sW2, 1, s + 1, 1);
         stage(sA2, sW2, sA3, sW3, 2, s + 2, 0);
         stage(sA3, sW3, sA0, sW0, 3, s + 3, 1);
       }
-      if (s < KS) stage(sA0, sW0, sA1, sW1, 0, s, 0);
-      if (s + 1 < KS) stage(sA1, sW1, sA2, sW2, 1, s + 1, 1);
-      if (s + 2 < KS) stage(sA2, sW2, sA3, sW3, 2, s + 2, 0);
+      if (s < most) stage(sA0, sW0, sA1, sW1, 0, s, 0);
+      if (s + 1 < most) stage(sA1, sW1, sA2, sW2, 1, s + 1, 1);
+      if (s + 2 < most) stage(sA2, sW2, sA3, sW3, 2, s + 2, 0);
+      if (KG > 1 && s + 3 < most) stage(sA3, sW3, sA0, sW0, 3, s + 3, 1);
     }
 
   };
@@ -763,22 +779,58 @@ __global__ __launch_bounds__(kThreads) void w4_ring_kernel(const GemmParams p, i
   } else {
     pipeline(std::integral_constant<int, MJ>{});
   }
+  if constexpr (KG > 1) {
+    // the second group's sums, through its own code stages, added to the first's
+    static_assert(KG == 2 && NI * MJ * 16 * 64 * 4 <= WB, "exchange region");
+    wait_copies_upto<0>();
+    __syncthreads();  // every wavefront is done with the stage buffers
+    float* ex = reinterpret_cast<float*>(wave == 0 ? sW0s : wave == 1 ? sW1s : wave == 2 ? sW2s : sW3s) + WB / 4 + lane;
+    if (kg == 1) {
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < MJ; ++j)
+#pragma unroll
+          for (int r = 0; r < 16; ++r) ex[((i * MJ + j) * 16 + r) * 64] = acc[i][j][r];
+    }
+    if (kg == 0) {
+      if (tid < BM) {
+        s_sx[tid] = 1.0f;
+        s_rw[tid] = e_rw;
+        s_yr[tid] = e_yr;
+      }
+      if (tid < BN) {
+        s_ws[tid] = 1.0f;
+        s_bs[tid] = e_bs;
+      }
+    }
+    __syncthreads();
+    if (kg == 1) return;
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < MJ; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[i][j][r] += ex[((i * MJ + j) * 16 + r) * 64];
+  }
   if (p.ksplit > 1) {
     tile_store_partials<BN, TN, TM, NI, MJ, ACT, false>(p, acc, row0, rows, n0, nlim, wn, wm, lane);
     return;
   }
-  wait_copies_upto<0>();
-  __syncthreads();  // every wavefront is done with the stage buffers
-  if (tid < BM) {
-    s_sx[tid] = 1.0f;
-    s_rw[tid] = e_rw;
-    s_yr[tid] = e_yr;
+  if constexpr (KG == 1) {
+    wait_copies_upto<0>();
+    __syncthreads();  // every wavefront is done with the stage buffers
+    if (tid < BM) {
+      s_sx[tid] = 1.0f;
+      s_rw[tid] = e_rw;
+      s_yr[tid] = e_yr;
+    }
+    if (tid < BN) {
+      s_ws[tid] = 1.0f;
+      s_bs[tid] = e_bs;
+    }
+    __syncthreads();
   }
-  if (tid < BN) {
-    s_ws[tid] = 1.0f;
-    s_bs[tid] = e_bs;
-  }
-  __syncthreads();
   // a wavefront's f32 region [32 tokens][TN rows]: an activation stage for
   // 64- and 128-token tiles, a code stage for 32-token tiles
   static_assert(32 * TN * 4 <= (BM >= 64 ? BM * 128 : BN * 32), "epilogue region");
@@ -813,13 +865,13 @@ void w4_launch_fmt(const GemmParams& p, int fmt, hipStream_t st) {
   else w4_launch_act<BM, KG, 0>(p, st);
 }
 
-template <int BM, int FMT>
+template <int BM, int KG, int FMT>
 void w4_launch_ring(const GemmParams& p, hipStream_t st) {
   const bool act = p.act != QA_NONE;
   const int n_tiles = cdiv(act ? p.N / 2 : p.N, act ? kW4BN / 2 : kW4BN), m_tiles = cdiv(p.M, BM);
   const dim3 grid(cdiv(m_tiles * n_tiles, kXcds) * kXcds, 1, (unsigned)std::max(1, p.ksplit));
-  if (act) hipLaunchKernelGGL((w4_ring_kernel<BM, true, FMT>), grid, dim3(kThreads), 0, st, p, m_tiles, n_tiles);
-  else hipLaunchKernelGGL((w4_ring_kernel<BM, false, FMT>), grid, dim3(kThreads), 0, st, p, m_tiles, n_tiles);
+  if (act) hipLaunchKernelGGL((w4_ring_kernel<BM, KG, true, FMT>), grid, dim3(KG * kThreads), 0, st, p, m_tiles, n_tiles);
+  else hipLaunchKernelGGL((w4_ring_kernel<BM, KG, false, FMT>), grid, dim3(KG * kThreads), 0, st, p, m_tiles, n_tiles);
 }
 
 // Dense NVFP4 / INT4 problems of at most 256 tokens whose 64-token tiles would
@@ -831,6 +883,12 @@ void w4_launch_ring(const GemmParams& p, hipStream_t st) {
 bool w4_ring(const GemmParams& p, int fmt, int n_tiles) {
   return fmt != 0 && !p.group_offs && p.M <= 256 && p.K <= 4096 && cdiv(p.M, 64) * n_tiles < 128;
 }
+
+// K groups per workgroup of the NVFP4 ring: two from 40 stages on, where their
+// halves outweigh the exchange at the end (one -> two groups, same K split,
+// 129 tokens: K 4096, N 4096 37.5 -> 32.4 us, K 2880, N 5760 27.3 -> 25.5; K
+// 2048, N 7168, 256 tokens 25.3 -> 26.6, K 512, N 8192 10.2 -> 11.4).
+int w4_ring_groups(const GemmParams& p) { return p.K >= 40 * 64 ? 2 : 1; }
 
 }  // namespace
 
@@ -866,12 +924,16 @@ bool qmoe_w4_plan(const GemmParams& p, int fmt, int* bm_out, int* ksplit_out, in
     // second one) and 696 in 128-token tiles, 32 rows 518 and 532
     bm = p.M / std::max(1, std::min(p.slots, p.M)) > 40 ? 128 : 64;
   } else if (w4_ring(p, fmt, n_tiles)) {
-    // (tile, split) measured best: NVFP4 32-token tiles, 4 slices up to 64
-    // tokens, 2 up to 128; INT4's costlier expansion keeps larger tiles
+    // (tile, split) measured best: NVFP4 32-token tiles in as many slices (up
+    // to 4, of at least 6 stages) as give every workgroup its own CU, XCD by
+    // XCD (K 4096, N 4096 at 65 / 129 / 203 tokens in 4 / 3 / 2 slices 17.9 /
+    // 22.5 / 28.6 us, in 2 / 1 / 1 22.4 / 32.4 / 33.4; K 1536, N 2000, 203
+    // tokens in 4 / 1 14.9 / 17.9; K 512, N 8192, 65 tokens in 1 / 2 9.9 /
+    // 12.0). INT4's costlier expansion keeps larger tiles
     const int tiles = cdiv(p.M, 64) * n_tiles;
     if (fmt == 1) {
       bm = 32;
-      ksplit = p.M <= 64 ? 4 : (p.M <= 128 ? 2 : 1);
+      ksplit = std::min({4, kCusPerXcd / cdiv(cdiv(p.M, 32) * n_tiles, kXcds), p.K / 64 / 6});
     } else if (p.M <= 128) {
       ksplit = std::min(cdiv(256, tiles), std::max(1, (p.K / 64) / 8));
     } else {
@@ -929,9 +991,9 @@ int qmoe_w4_launch(GemmParams p, int fmt, void* workspace, int64_t ws_bytes, hip
   }
   const int n_tiles = cdiv(p.act != QA_NONE ? p.N / 2 : p.N, p.act != QA_NONE ? kW4BN / 2 : kW4BN);
   if (w4_ring(p, fmt, n_tiles)) {
-    if (fmt == 1) w4_launch_ring<32, 1>(p, st);
-    else if (bm == 128) w4_launch_ring<128, 2>(p, st);
-    else w4_launch_ring<64, 2>(p, st);
+    if (fmt == 1) w4_ring_groups(p) == 2 ? w4_launch_ring<32, 2, 1>(p, st) : w4_launch_ring<32, 1, 1>(p, st);
+    else if (bm == 128) w4_launch_ring<128, 1, 2>(p, st);
+    else w4_launch_ring<64, 1, 2>(p, st);
   } else if (bm == 128) {
     // two K groups of wavefronts per workgroup where one workgroup per CU is all there is
     if (p.group_offs || cdiv(p.M, 128) * n_tiles * ksplit > 256) w4_launch_fmt<128, 1>(p, fmt, st);
