@@ -67,14 +67,22 @@ __device__ __forceinline__ void wait_copies_upto() {
 // does not order it against the LDS reads: it would drain every copy in
 // flight before a read of a ring buffer whose index it cannot resolve. The
 // kernel's own counted waits and barriers order them. The instruction has no
-// register result and takes its address registers when it issues; the
-// s_nop is the wait state between a write of M0 and its use. A kernel that
-// uses these makes no other use of M0 (no copy builtins beside them).
+// register result and takes its address registers when it issues. The
+// compiler adds no wait states inside assembly: the instruction between the
+// write of M0 and the copy is the one that M0 needs. A vector-memory read of a
+// scalar register needs five after a vector instruction wrote it, and the
+// compiler may put a v_readfirstlane of `base` right before the assembly; the
+// scalar move of `base` waits for that by itself, and the copy for the move.
+// A kernel that uses these makes no other use of M0 (no copy builtins beside
+// them).
 __device__ __forceinline__ void lds_copy16(const uint8_t* src, uint32_t lds) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
 }
 __device__ __forceinline__ void lds_copy16(const uint8_t* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
+  const uint8_t* b;
+  asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
+               : "=&s"(b)
+               : "s"(lds), "v"(off), "s"(base)
                : "memory");
 }
 // The same for 4 bytes per lane (`lds` + 4 * lane).
