@@ -54,6 +54,21 @@ def _violations(lines):
     return found
 
 
+def test_assembly_that_writes_m0_says_so():
+    """The compiler keeps its own values in M0 (LDS copies, indexed moves) and
+    reads nothing in an assembly text: the clobber list has to name it."""
+    from qmoe import build
+
+    checked = 0
+    for name in sorted(os.listdir(build.CSRC)):
+        with open(os.path.join(build.CSRC, name)) as f:
+            for stmt in re.findall(r"\basm\b[^;]*;", f.read()):
+                if re.search(r"s_mov_b32 m0", stmt):
+                    checked += 1
+                    assert re.search(r':[^:]*"m0"[^:]*\)\s*;$', stmt), f"{name}: {stmt}"
+    assert checked >= 3
+
+
 def test_scan_finds_a_short_wait():
     """The scan itself, on text with and without the wait states."""
     k = ["0000 <k>:", "\tv_readfirstlane_b32 s2, v1 // 00: 00"]

@@ -73,21 +73,19 @@ __device__ __forceinline__ void wait_copies_upto() {
 // scalar register needs five after a vector instruction wrote it, and the
 // compiler may put a v_readfirstlane of `base` right before the assembly; the
 // scalar move of `base` waits for that by itself, and the copy for the move.
-// A kernel that uses these makes no other use of M0 (no copy builtins beside
-// them).
 __device__ __forceinline__ void lds_copy16(const uint8_t* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "m0", "memory");
 }
 __device__ __forceinline__ void lds_copy16(const uint8_t* base, uint32_t off, uint32_t lds) {
   const uint8_t* b;
   asm volatile("s_mov_b32 m0, %1\n\ts_mov_b64 %0, %3\n\tglobal_load_lds_dwordx4 %2, %0"
                : "=&s"(b)
                : "s"(lds), "v"(off), "s"(base)
-               : "memory");
+               : "m0", "memory");
 }
 // The same for 4 bytes per lane (`lds` + 4 * lane).
 __device__ __forceinline__ void lds_copy4(const void* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(src) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds), "v"(src) : "m0", "memory");
 }
 
 template <int BM>
