@@ -69,12 +69,7 @@ __global__ __launch_bounds__(kT8Threads, 2) void t8_gemm_kernel(const GemmParams
 
   int g, row0, rows, ntile;
   if (p.group_offs) {
-    // XCD x walks the m-tiles x, x + 8, ..., all weight tiles of one before
-    // the next (an m-tile's activation rows come from one L2)
-    const int slot = blockIdx.x / kXcds;
-    ntile = slot % n_tiles;
-    if (!tile_group<BM>(p, slot / n_tiles * kXcds + blockIdx.x % kXcds, g, row0, rows, reinterpret_cast<int*>(smem)))
-      return;
+    if (!tile_group_xcd<BM>(p, blockIdx.x, n_tiles, g, row0, rows, ntile, reinterpret_cast<int*>(smem))) return;
     __syncthreads();  // the group has been read everywhere: the buffers are free
   } else {
     int mt;
@@ -402,8 +397,8 @@ __global__ __launch_bounds__(kT8Threads, 2) void t8_gemm_kernel(const GemmParams
 template <bool F8, int BM, bool ACT, bool WPC, int WF = 0>
 void t8_launch_shape(const GemmParams& p, hipStream_t st) {
   const int n_tiles = cdiv(ACT ? p.N / 2 : p.N, ACT ? kT8BN / 2 : kT8BN);
-  const int m_tiles = p.group_offs ? cdiv(cdiv(p.M, BM) + std::min(p.slots, p.M), kXcds) * kXcds : cdiv(p.M, BM);
-  const int grid = p.group_offs ? m_tiles * n_tiles : cdiv(m_tiles * n_tiles, kXcds) * kXcds;
+  const int m_tiles = cdiv(p.M, BM) + (p.group_offs ? std::min(p.slots, p.M) : 0);
+  const int grid = cdiv(m_tiles * n_tiles, kXcds) * kXcds;
   hipLaunchKernelGGL((t8_gemm_kernel<F8, BM, ACT, WPC, WF>), dim3(grid), dim3(kT8Threads), 0, st, p, m_tiles, n_tiles);
 }
 

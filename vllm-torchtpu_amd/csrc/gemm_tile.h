@@ -133,6 +133,88 @@ __device__ __forceinline__ bool tile_group(const GemmParams& p, int y, int& g, i
   return g >= 0;
 }
 
+// Grouped tile of a 1-D grid (the groups' m-tiles, found by a scan of their
+// sizes, times n_tiles weight tiles). XCD x takes the m-tiles x, x + 8, ...,
+// all weight tiles of one before the next, so that an m-tile's activation rows
+// come from one L2, while the m-tiles of an expert read its weights at the
+// same time on their XCDs. The weight tiles of the m-tiles left over when
+// fewer than 8 remain are dealt evenly to all XCDs: with these dealt whole too,
+// few m-tiles left XCDs idle (MXFP4, K 2880, N 2880: 8 experts, 512 tokens 81
+// -> 58 us; 64 experts, 16 tokens 54 -> 34). In one contiguous run of m-tiles
+// per XCD an expert's weights are read again for each of its m-tiles (FP8, 8
+// experts, K 4096, N 28672, 300 rows each: 515 -> 612 us). Block b is number
+// b / 8 of XCD b % 8; those past its end return false. One wavefront reads
+// four groups per lane, so that up to 256 groups cost one memory latency.
+// s_info: four ints of LDS.
+template <int BM>
+__device__ __forceinline__ bool tile_group_xcd(const GemmParams& p, int b, int n_tiles, int& g, int& row0, int& rows,
+                                               int& ntile, int* s_info) {
+  constexpr int kPer = 4, kChunk = 64 * kPer;
+  if (threadIdx.x < 64) {
+    const int lane = threadIdx.x, G = p.slots;
+    int o[kPer + 1], nt[kPer], incl = 0, sum = 0;
+    auto read_chunk = [&](int c0) {  // groups c0 + 4 lane ..: rows, m-tiles, their scan
+      sum = 0;
+#pragma unroll
+      for (int i = 0; i <= kPer; ++i) o[i] = p.group_offs[min(c0 + lane * kPer + i, G)];
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        nt[i] = (o[i + 1] - o[i] + BM - 1) / BM;
+        sum += nt[i];
+      }
+      incl = sum;
+#pragma unroll
+      for (int d = 1; d < 64; d <<= 1) {
+        const int v = __shfl_up(incl, d, 64);
+        if (lane >= d) incl += v;
+      }
+    };
+    int total = 0;
+    for (int c0 = 0; c0 < G; c0 += kChunk) {
+      read_chunk(c0);
+      total += __shfl(incl, 63, 64);
+    }
+    const int xcd = b % kXcds, slot = b / kXcds, whole = total / kXcds * n_tiles;
+    int y, nt_of;  // m-tile and weight tile of the block
+    bool mine = true;
+    if (slot < whole) {
+      y = slot / n_tiles * kXcds + xcd;
+      nt_of = slot % n_tiles;
+    } else {
+      const int left = total % kXcds * n_tiles, per = (left + kXcds - 1) / kXcds;
+      const int pair = xcd * per + slot - whole;
+      mine = slot - whole < per && pair < left;
+      y = total / kXcds * kXcds + pair / n_tiles;
+      nt_of = pair % n_tiles;
+    }
+    if (!mine) {
+      if (lane == 0) s_info[0] = -1;
+    } else {
+      for (int c0 = 0; c0 < G; c0 += kChunk) {
+        if (G > kChunk) read_chunk(c0);
+        int t = y - (incl - sum);  // counted from the lane's first m-tile
+#pragma unroll
+        for (int i = 0; i < kPer; ++i) {
+          if (t >= 0 && t < nt[i]) {  // one lane of one chunk
+            s_info[0] = c0 + lane * kPer + i;
+            s_info[1] = o[i] + t * BM;
+            s_info[2] = min(BM, o[i + 1] - o[i] - t * BM);
+            s_info[3] = nt_of;
+          }
+          t -= nt[i];
+        }
+        y -= __shfl(incl, 63, 64);  // from the next chunk's first
+      }
+    }
+  }
+  __syncthreads();
+  g = __builtin_amdgcn_readfirstlane(s_info[0]);
+  row0 = __builtin_amdgcn_readfirstlane(s_info[1]);
+  rows = __builtin_amdgcn_readfirstlane(s_info[2]);
+  ntile = __builtin_amdgcn_readfirstlane(s_info[3]);
+  return g >= 0;
+}
+
 __device__ __forceinline__ bool tile_dense(int b, int m_tiles, int n_tiles, int& mt, int& nt) {
   const int total = m_tiles * n_tiles;
   const int per = (total + kXcds - 1) / kXcds;

@@ -109,13 +109,7 @@ __global__ __launch_bounds__(KG * kThreads, 2) void w4_gemm_kernel(const GemmPar
 
   int g, row0, rows, ntile;
   if (p.group_offs) {
-    // consecutive workgroups go round-robin to the XCDs: XCD x walks the
-    // m-tiles x, x + 8, ..., all weight tiles of one before the next, so
-    // that an m-tile's activation rows come from one L2
-    const int slot = blockIdx.x / kXcds;
-    ntile = slot % n_tiles;
-    if (!tile_group<BM>(p, slot / n_tiles * kXcds + blockIdx.x % kXcds, g, row0, rows, reinterpret_cast<int*>(smem_all)))
-      return;
+    if (!tile_group_xcd<BM>(p, blockIdx.x, n_tiles, g, row0, rows, ntile, reinterpret_cast<int*>(smem_all))) return;
     __syncthreads();  // the group has been read everywhere: the buffers are free
   } else {
     int mt;
@@ -846,8 +840,8 @@ void w4_launch_shape(const GemmParams& p, hipStream_t st) {
   const int nout = ACT ? p.N / 2 : p.N;
   const int n_tiles = cdiv(nout, ACT ? kW4BN / 2 : kW4BN);
   const unsigned ks = (unsigned)std::max(1, p.ksplit);
-  const int m_tiles = p.group_offs ? cdiv(cdiv(p.M, BM) + std::min(p.slots, p.M), kXcds) * kXcds : cdiv(p.M, BM);
-  const int grid = p.group_offs ? m_tiles * n_tiles : cdiv(m_tiles * n_tiles, kXcds) * kXcds;
+  const int m_tiles = cdiv(p.M, BM) + (p.group_offs ? std::min(p.slots, p.M) : 0);
+  const int grid = cdiv(m_tiles * n_tiles, kXcds) * kXcds;
   hipLaunchKernelGGL((w4_gemm_kernel<BM, KG, ACT, FMT>), dim3(grid, 1, ks), dim3(KG * kThreads), 0, st, p, m_tiles,
                      n_tiles);
 }
