@@ -66,14 +66,48 @@ def test_dense(monkeypatch, fmt, K, pad, M, N):
 
 
 @pytest.mark.parametrize("fmt", ["mx", "nv", "i4"])
+@pytest.mark.parametrize("bm,M,N,K,act", [
+    (32, 257, 700, 576, None), (64, 300, 700, 1088, None), (128, 400, 515, 320, None),  # two K groups
+    (64, 1100, 4000, 128, None), (128, 2049, 4000, 192, None),  # 288 and 272 tiles: one K group
+    (32, 70, 1000, 320, "silu"), (64, 129, 1000, 576, "swigluoai"), (128, 300, 514, 192, "silu"),
+    (128, 2049, 4000, 128, "silu"),  # 17 x 16 tiles of gate and up rows
+])
+def test_dense_line_tiles(monkeypatch, fmt, bm, M, N, K, act):
+    """Every instance of the line pipeline in dense problems: tile heights,
+    one and two K groups, fused activations, ragged channels and tokens."""
+    from qmoe import ops
+
+    gen = torch.Generator(device="cuda").manual_seed(K + M + N)
+    codes, s, val = _weights(fmt, N, K, 0, gen)
+    x = torch.randn((M, K), device="cuda", generator=gen).to(torch.bfloat16)
+    h, mag = x.double() @ val.t(), x.double().abs() @ val.abs().t()
+    if act:
+        g, u = h[:, :N // 2], h[:, N // 2:]
+        # |d act| <= 2 |u| dg + 2 |g| du near these sizes
+        mag = 2 * ((u.abs() + 1) * mag[:, :N // 2] + (g.abs() + 1) * mag[:, N // 2:]) + 1
+        if act == "silu":
+            h = g * torch.sigmoid(g) * u
+        else:
+            g, u = g.clamp(max=7.0), u.clamp(-7.0, 7.0)
+            h = (u + 1) * g * torch.sigmoid(1.702 * g)
+    monkeypatch.setenv("QMOE_SKINNY_MAX_ROWS", "0")
+    monkeypatch.setenv("QMOE_SKINNY_ROW_SPLIT", "0")
+    monkeypatch.setenv("QMOE_W4_BM", str(bm))
+    for ks in (1, 2) if K >= 320 else (1,):
+        monkeypatch.setenv("QMOE_W4_KSPLIT", str(ks))
+        with ops.record_plans() as plans:
+            got = ops.gemm(_kind(fmt), x, codes, w_scale=s, activation=act)
+        assert tuple(plans[0][4:]) == ("tiled_4b", bm, ks)
+        _check(got, h, mag)
+
+
+@pytest.mark.parametrize("fmt", ["mx", "nv", "i4"])
 @pytest.mark.parametrize("bm", ["64", "128"])
 @pytest.mark.parametrize("K,N,act", [(320, 64, None), (576, 520, "silu"), (1088, 514, "swigluoai"), (2880, 256, None)])
 def test_grouped(monkeypatch, fmt, bm, K, N, act):
     """Experts of 0, 1, 31, 33, 65, 96, 97 and 140 rows, gathered tokens, scattered rows, weights and bias."""
     from qmoe import ops
 
-    if fmt == "i4" and act == "swigluoai":
-        pytest.skip("as the other formats")
     gen = torch.Generator(device="cuda").manual_seed(K + N)
     counts = [0, 1, 31, 33, 65, 96, 97, 140]
     E, M, T = len(counts), sum(counts), 90

@@ -1,0 +1,71 @@
+"""Which kernel, tile and K split a problem gets (no GPU: the plans read no
+memory), on both sides of the rules' lines."""
+
+import ctypes
+
+import pytest
+
+
+def _plan(kind, M, N, K, **kw):
+    from qmoe import _capi, ops
+
+    if kind == "W4A16_I4":
+        kw["wq_group"] = 32
+    return ops.plan_for_shape(getattr(_capi, kind), M, N, K, **kw)[4:]
+
+
+@pytest.mark.parametrize("kind,M,N,K,tile,ks", [
+    # one round of 64-token tiles, two workgroups per CU, before 128-token tiles on half of the CUs
+    ("W4A16_MX", 700, 5760, 2880, 64, 1),
+    ("W4A16_NV", 700, 5760, 2880, 64, 1),
+    ("W4A16_I4", 700, 5760, 2880, 64, 1),
+    ("W4A16_MX", 4096, 5760, 2880, 128, 1),  # more than a round of them
+    ("W4A16_MX", 512, 32768, 512, 128, 1),
+    # few tiles over a long K: more than four slices
+    ("W4A16_MX", 128, 256, 7168, 32, 12),
+    ("W4A16_NV", 128, 256, 7168, 32, 12),
+    ("W4A16_I4", 128, 256, 7168, 32, 12),
+    ("W4A16_I4", 1024, 128, 2880, 32, 8),
+    ("W4A16_NV", 203, 5760, 2880, 32, 1),
+    # tiles in multiples of the XCDs: 84 tiles in 3 slices would be 264 workgroups
+    ("W4A16_MX", 65, 7168, 2048, 32, 2),
+    ("W4A16_MX", 33, 256, 64, 32, 1),  # a single stage
+])
+def test_dense_4bit_plans(monkeypatch, kind, M, N, K, tile, ks):
+    monkeypatch.setenv("QMOE_SKINNY_ROW_SPLIT", "0")
+    monkeypatch.setenv("QMOE_SKINNY_MAX_ROWS", "0")
+    assert _plan(kind, M, N, K) == ("tiled_4b", tile, ks)
+
+
+@pytest.mark.parametrize("kind", ["W4A16_MX", "W4A16_NV", "W4A16_I4"])
+@pytest.mark.parametrize("M", [33, 100, 256, 257, 2000, 8192])
+@pytest.mark.parametrize("N", [1, 255, 1000, 5760])
+def test_dense_4bit_workspace_is_bounded(monkeypatch, kind, M, N):
+    """A split is one workgroup per CU: its f32 slices are at most 256 tiles."""
+    from qmoe import _capi
+
+    monkeypatch.setenv("QMOE_SKINNY_MAX_ROWS", "0")
+    monkeypatch.setenv("QMOE_SKINNY_ROW_SPLIT", "0")
+    for K in (64, 320, 2880, 16384):
+        path, tile, ks = _plan(kind, M, N, K)
+        assert path == "tiled_4b" and ks >= 1 and (ks == 1 or K // 64 // ks >= 4)
+        if ks > 1:
+            tiles = -(-M // tile) * -(-N // 256)
+            assert tiles * ks <= 256 and ks * M * N * 4 <= 256 * tile * 256 * 4 <= 64 << 20
+        d = _capi.GemmDesc()
+        d.kind, d.a, d.w, d.y, d.w_scale = getattr(_capi, kind), 1 << 24, 1 << 24, 1 << 24, 1 << 24
+        d.lda, d.ldw, d.ldy, d.ldws = K, K // 2, N, K // (16 if kind == "W4A16_NV" else 32)
+        d.M, d.N, d.K, d.slots, d.max_rows, d.wq_group = M, N, K, 1, M, 32 if kind == "W4A16_I4" else 0
+        n = ctypes.c_int64(0)
+        assert _capi.lib.qmoe_gemm_workspace_size(ctypes.byref(d), ctypes.byref(n)) == 0
+        assert n.value == (ks * M * N * 4 if ks > 1 else 0)
+
+
+@pytest.mark.parametrize("bm", [32, 64, 128])
+@pytest.mark.parametrize("kind,M", [("W4A16_MX", 129), ("W4A16_NV", 129), ("W4A16_I4", 100), ("W4A16_NV", 700)])
+def test_forced_4bit_tile_height(monkeypatch, bm, kind, M):
+    monkeypatch.setenv("QMOE_SKINNY_MAX_ROWS", "0")
+    monkeypatch.setenv("QMOE_W4_BM", str(bm))
+    assert _plan(kind, M, 5760, 2880) == ("tiled_4b", bm, 1)
+    monkeypatch.setenv("QMOE_W4_KSPLIT", "3")
+    assert _plan(kind, M, 5760, 2880) == ("tiled_4b", bm, 3)

@@ -55,7 +55,6 @@ namespace {
 
 using rsrc_t = __amdgpu_buffer_rsrc_t;
 constexpr int kW4BN = 256;  // weight rows per tile
-constexpr int kCusPerXcd = 32;
 
 __device__ __forceinline__ int w4_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
@@ -513,17 +512,15 @@ struct W4Shape {
   static_assert(NI >= 1 && MJ >= 1, "tile too small");
 };
 
-// Short under-filled dense problems of the costlier formats (1 NVFP4, 2 INT4;
-// w4_ring below has the rule): one workgroup per tile whose stages of 64 k --
+// Under-filled dense problems of the costlier formats (1 NVFP4, 2 INT4;
+// w4_plan_dense has the rule): one workgroup per tile whose stages of 64 k --
 // activations, codes and scales alike -- run through a ring of four, copied
 // four stages ahead, with the operand reads and copies of a stage spread
 // over its MFMAs. It spends fewer instructions per stage than the line
 // pipeline above, and with one workgroup per CU that is what counts: NVFP4 K
-// 2880, N 5760 at 128 / 203 tokens 22.6 / 27.7 us against 26.0 / 32.0. What
-// bounds it is the expansion, about 1500 cycles per stage on the vector ALU:
-// two K groups of four wavefronts (KG 2, their sums added through LDS) shorten
-// a long chain of stages by a few percent only (203 tokens 28.6 -> 27.7 us, K
-// 4096, N 4096 38.3 -> 33.1), the K split the rest (28.6).
+// 2880, N 5760 at 128 / 203 tokens 22.6 / 27.7 us against 26.0 / 32.0. The
+// expansion bounds it: two K groups of four wavefronts (KG 2, their sums added
+// through LDS) take 0.84 us per stage of each, one alone 0.50.
 template <int BM, int KG, bool ACT, int FMT>
 __global__ __launch_bounds__(KG * kThreads) void w4_ring_kernel(const GemmParams p, int m_tiles, int n_tiles) {
   constexpr bool NV = FMT == 1, I4 = FMT == 2;
@@ -548,14 +545,9 @@ __global__ __launch_bounds__(KG * kThreads) void w4_ring_kernel(const GemmParams
   const int lane = tid & 63, wave = tid >> 6;
   const int wn = wave % S::WN, wm = wave / S::WN;
 
-  int g, row0, rows, ntile;
-  {
-    int mt;
-    if (!tile_dense(blockIdx.x, m_tiles, n_tiles, mt, ntile)) return;
-    g = 0;
-    row0 = mt * BM;
-    rows = min(BM, p.M - row0);
-  }
+  int mt, ntile;
+  if (!tile_dense(blockIdx.x, m_tiles, n_tiles, mt, ntile)) return;
+  const int row0 = mt * BM, rows = min(BM, p.M - row0);
   const int n0 = ntile * BNO;
   const int nlim = ACT ? p.N / 2 : p.N;
   // global weight row of tile LDS row r (gate rows, then up rows with ACT);
@@ -574,7 +566,7 @@ __global__ __launch_bounds__(KG * kThreads) void w4_ring_kernel(const GemmParams
     if (p.row_weight) e_rw = bf16_to_f32(p.row_weight[R]);
     e_yr = p.y_rows ? p.y_rows[R] : R;
   }
-  if (tid < BN && p.bias) e_bs = p.bias[(int64_t)g * p.bias_gstride + wrow_global(tid)];
+  if (tid < BN && p.bias) e_bs = p.bias[wrow_global(tid)];
 
   // ---- LDS copies (16 bytes per lane) ----
   // activations: one instruction = 8 rows x 128 bytes (lane -> row l >> 3,
@@ -588,9 +580,9 @@ __global__ __launch_bounds__(KG * kThreads) void w4_ring_kernel(const GemmParams
   constexpr int XI = BM / 32;  // activation copies per wavefront
   constexpr int WI = 2;        // code copies per wavefront
   const uint8_t* xbase = static_cast<const uint8_t*>(p.a);
-  const uint8_t* wbase = p.w + (int64_t)g * p.w_gstride;
+  const uint8_t* wbase = p.w;
   const rsrc_t eres = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<void*>(static_cast<const void*>(static_cast<const uint8_t*>(p.w_scale) + (int64_t)g * p.ws_gstride * kSB)),
+      const_cast<void*>(static_cast<const void*>(p.w_scale)),
       (short)0, (int)std::min<int64_t>((int64_t)p.N * p.ldws * kSB, 0x7fffffff), 0x00020000);
   const uint64_t lda_b = (uint64_t)p.lda * 2;
   uint32_t xrow[XI], woff[WI];
@@ -758,16 +750,11 @@ __global__ __launch_bounds__(KG * kThreads) void w4_ring_kernel(const GemmParams
     }
 
   };
-  // A tile with at most 32 (64) valid tokens -- a routed expert's last tile
-  // -- runs the MFMAs of its first one (two) 32-token blocks only: the
-  // others' sums belong to no token. The expansion of the weight codes, the
-  // copies and the barriers are the same.
+  // A 64-token tile with at most 32 valid tokens runs the MFMAs of its first
+  // 32-token block only: the others' sums belong to no token. The expansion of
+  // the weight codes, the copies and the barriers are the same.
   const int rows_u = __builtin_amdgcn_readfirstlane(rows);
-  if constexpr (MJ == 4) {
-    if (rows_u <= 32) pipeline(std::integral_constant<int, 1>{});
-    else if (rows_u <= 64) pipeline(std::integral_constant<int, 2>{});
-    else pipeline(std::integral_constant<int, 4>{});
-  } else if constexpr (MJ == 2) {
+  if constexpr (MJ == 2) {
     if (rows_u <= 32) pipeline(std::integral_constant<int, 1>{});
     else pipeline(std::integral_constant<int, 2>{});
   } else {
@@ -826,7 +813,7 @@ __global__ __launch_bounds__(KG * kThreads) void w4_ring_kernel(const GemmParams
     __syncthreads();
   }
   // a wavefront's f32 region [32 tokens][TN rows]: an activation stage for
-  // 64- and 128-token tiles, a code stage for 32-token tiles
+  // 64-token tiles, a code stage for 32-token tiles
   static_assert(32 * TN * 4 <= (BM >= 64 ? BM * 128 : BN * 32), "epilogue region");
   uint8_t* regb;
   if constexpr (BM >= 64) regb = wave == 0 ? sA0 : wave == 1 ? sA1 : wave == 2 ? sA2 : sA3;
@@ -868,30 +855,109 @@ void w4_launch_ring(const GemmParams& p, hipStream_t st) {
   else hipLaunchKernelGGL((w4_ring_kernel<BM, KG, false, FMT>), grid, dim3(KG * kThreads), 0, st, p, m_tiles, n_tiles);
 }
 
-// Dense NVFP4 / INT4 problems of at most 256 tokens whose 64-token tiles would
-// leave half of the CUs idle and whose K is too short to split: the ring
-// kernel. Measured on MI355X, NVFP4: K 2880, N 5760 at 128 / 203 tokens 23.4 /
-// 28.1 us against 26.0 / 32.0; with 224 such tiles (N 14336, K 4096, 203
-// tokens) the line pipeline takes 52.5 us against 70.9, with K 14336, N 4096
-// 52.7 against 136.
-bool w4_ring(const GemmParams& p, int fmt, int n_tiles) {
-  return fmt != 0 && !p.group_offs && p.M <= 256 && p.K <= 4096 && cdiv(p.M, 64) * n_tiles < 128;
+// The kernel of a problem: token-tile height, K groups of wavefronts per
+// workgroup, K slices, and whether the ring kernel runs it.
+struct W4Plan {
+  int bm = 128, kgroups = 1, ksplit = 1;
+  bool ring = false;
+};
+
+// One round of workgroups on MI355X takes `start` + `stage` us per 64-k stage
+// of a K group, by kernel and format (MXFP4, NVFP4, INT4). Fitted to 171 dense
+// problems per format (K 512..14336, N 128..32768, 65..4096 tokens, one to 12
+// slices), which they meet within 8 % (rms).
+struct W4Time {
+  int bm, kgroups;
+  bool ring;
+  float start[3], stage[3];
+};
+constexpr W4Time kW4Times[] = {
+    {32, 2, false, {6.7f, 7.5f, 8.0f}, {0.63f, 1.07f, 1.29f}},
+    {64, 2, false, {9.4f, 10.0f, 10.3f}, {0.87f, 1.25f, 1.47f}},
+    {128, 2, false, {13.4f, 13.8f, 14.0f}, {1.34f, 1.68f, 1.93f}},
+    {64, 1, false, {9.7f, 9.9f, 10.4f}, {0.90f, 1.26f, 1.44f}},
+    {128, 1, false, {9.2f, 8.5f, 9.3f}, {1.51f, 1.84f, 2.09f}},
+    {32, 1, true, {0, 6.0f, 0}, {0, 0.50f, 0}},
+    {32, 2, true, {0, 7.6f, 0}, {0, 0.84f, 0}},
+    {64, 1, true, {0, 0, 7.9f}, {0, 0, 0.77f}},
+};
+
+// Dense problems of more than one round of 64-token tiles (two workgroups of
+// one K group per CU) take 128-token tiles (64-token ones lose 5 to 30 % from
+// there on). The others take the kernel and K split of the least time: two K
+// groups where the workgroups fill only one per CU, one group above that; a
+// split only within one workgroup per CU, which also bounds its f32 slices to
+// 256 tiles; the ring kernel up to 256 tokens. The XCDs are dealt whole tiles,
+// so a count is rounded up to 8. The ring ends at K 8192 (NVFP4 K 14336, N
+// 4096, 129 tokens 56.6 us, the line kernel 46.6). Measured against the rules
+// before (the largest tiles on at least 130 CUs, at most 4 slices of at least
+// 28 stages, the ring up to K 4096): MXFP4 / NVFP4 / INT4 4 / 6 / 9 % faster
+// over 192 problems, e.g. K 2880, N 5760, 700 tokens 46.5 / 57.0 / 61.6 -> 31.6 / 41.6 / 46.1 us,
+// NVFP4 / INT4 K 7168, N 256, 128 tokens 24.9 / 29.0 -> 15.9 / 20.4.
+W4Plan w4_plan_dense(const GemmParams& p, int fmt, int n_tiles, int force_bm, int force_ks) {
+  const int nu = p.K / 64;
+  auto workgroups = [&](int bm, int ks) { return cdiv<int64_t>((int64_t)cdiv(p.M, bm) * n_tiles, kXcds) * kXcds * ks; };
+  W4Plan best;
+  if (force_bm) {
+    best.bm = force_bm;
+    best.ksplit = std::max(force_ks, 1);
+    best.kgroups = force_bm == 32 || workgroups(force_bm, best.ksplit) <= 256 ? 2 : 1;
+    return best;
+  }
+  if (!force_ks && workgroups(64, 1) > 512) return best;
+  float best_us = -1.0f;
+  for (int k : {1, 2, 3, 4, 6, 8, 12}) {
+    const int ks = force_ks ? force_ks : k;
+    if (!force_ks && ks > 1 && nu / ks < 4) break;
+    for (const W4Time& t : kW4Times) {
+      if (t.ring && (t.start[fmt] == 0 || p.M > 256 || p.K > 8192)) continue;
+      const int64_t n = workgroups(t.bm, ks), round = t.kgroups == 1 && !t.ring ? 512 : 256;
+      if (round == 512 && n <= 256) continue;  // one workgroup per CU: two K groups
+      if (!force_ks && n > (ks > 1 ? 256 : t.bm == 32 && !t.ring ? 512 : round)) continue;
+      float us = (float)cdiv(n, round) * (t.start[fmt] + t.stage[fmt] * (float)cdiv(cdiv(nu, ks), t.kgroups));
+      if (ks > 1) us += 2.5f + 0.4e-6f * (float)((int64_t)p.M * p.N * 4 * ks);  // the finishing launch and its slices
+      if (best_us < 0 || us < best_us) {
+        best_us = us;
+        best.bm = t.bm;
+        best.kgroups = t.kgroups;
+        best.ksplit = ks;
+        best.ring = t.ring;
+      }
+    }
+    if (force_ks) break;
+  }
+  return best;
 }
 
-// K groups per workgroup of the NVFP4 ring: two from 40 stages on, where their
-// halves outweigh the exchange at the end (one -> two groups, same K split,
-// 129 tokens: K 4096, N 4096 37.5 -> 32.4 us, K 2880, N 5760 27.3 -> 25.5; K
-// 2048, N 7168, 256 tokens 25.3 -> 26.6, K 512, N 8192 10.2 -> 11.4).
-int w4_ring_groups(const GemmParams& p) { return p.K >= 40 * 64 ? 2 : 1; }
+// Routed experts, measured on MI355X (GPT-OSS MoE, 128 experts, MXFP4): 64
+// rows per routed expert 797 us in 64-token tiles (half of the experts need a
+// second one) and 696 in 128-token tiles, 32 rows 518 and 532.
+W4Plan w4_plan_grouped(const GemmParams& p, int force_bm, int force_ks) {
+  W4Plan r;
+  if (force_bm) r.bm = std::max(force_bm, 64);
+  else r.bm = p.M / std::max(1, std::min(p.slots, p.M)) > 40 ? 128 : 64;
+  r.ksplit = std::max(force_ks, 1);
+  return r;
+}
+
+// The plan of a problem that the kernels take (qmoe_w4_plan checks that).
+// QMOE_W4_BM forces the line kernel in that tile height, QMOE_W4_KSPLIT the K
+// split (tuning knobs).
+W4Plan w4_choose(const GemmParams& p, int fmt, int n_tiles) {
+  const char* env = getenv("QMOE_W4_BM");
+  const int bm = env && (atoi(env) == 128 || atoi(env) == 64 || atoi(env) == 32) ? atoi(env) : 0;
+  const char* ks_env = getenv("QMOE_W4_KSPLIT");
+  const int ks = ks_env && atoi(ks_env) > 0 ? std::min(atoi(ks_env), p.K / 64) : 0;
+  return p.group_offs ? w4_plan_grouped(p, bm, ks) : w4_plan_dense(p, fmt, n_tiles, bm, ks);
+}
 
 }  // namespace
 
-// Whether the W4A16 tiled kernel takes the problem (K % 64, 16-byte aligned
+// Whether the W4A16 tiled kernels take the problem (K % 64, 16-byte aligned
 // rows, even scale rows, codes < 4 GiB per group), and its plan: token-tile
-// height (the largest of 128 / 64 / 32 that still fills the CUs, or that fits
-// the average group), K split (dense problems with few tiles) and the f32
-// workspace the split needs ([ksplit][M][N]). `fmt`: 0 MXFP4 (e8m0 per
-// 32 k), 1 NVFP4 (bf16 per 16 k), 2 INT4 (bf16 per wq_group k).
+// height, K split and the f32 workspace the split needs ([ksplit][M][N]).
+// `fmt`: 0 MXFP4 (e8m0 per 32 k), 1 NVFP4 (bf16 per 16 k), 2 INT4 (bf16 per
+// wq_group k).
 bool qmoe_w4_plan(const GemmParams& p, int fmt, int* bm_out, int* ksplit_out, int64_t* ws_bytes) {
   if (p.M <= 0 || p.K <= 0 || (p.K % 64) != 0 || p.N <= 0) return false;
   if (p.act != QA_NONE && (p.N % 2) != 0) return false;
@@ -908,64 +974,10 @@ bool qmoe_w4_plan(const GemmParams& p, int fmt, int* bm_out, int* ksplit_out, in
     return false;
   const int nout = p.act != QA_NONE ? p.N / 2 : p.N;
   const int n_tiles = cdiv(nout, p.act != QA_NONE ? kW4BN / 2 : kW4BN);
-  int bm = 64, ksplit = 1;
-  const char* env = getenv("QMOE_W4_BM");  // tuning knob
-  if (env && (atoi(env) == 128 || atoi(env) == 64 || atoi(env) == 32)) {
-    bm = p.group_offs && atoi(env) == 32 ? 64 : atoi(env);
-  } else if (p.group_offs) {
-    // measured on MI355X (GPT-OSS MoE, 128 experts, MXFP4): 64 rows per
-    // routed expert 797 us in 64-token tiles (half of the experts need a
-    // second one) and 696 in 128-token tiles, 32 rows 518 and 532
-    bm = p.M / std::max(1, std::min(p.slots, p.M)) > 40 ? 128 : 64;
-  } else if (w4_ring(p, fmt, n_tiles)) {
-    // (tile, split) measured best: NVFP4 32-token tiles in as many slices (up
-    // to 4, of at least 6 stages) as give every workgroup its own CU, XCD by
-    // XCD (K 4096, N 4096 at 65 / 129 / 203 tokens in 4 / 3 / 2 slices 17.9 /
-    // 22.5 / 28.6 us, in 2 / 1 / 1 22.4 / 32.4 / 33.4; K 1536, N 2000, 203
-    // tokens in 4 / 1 14.9 / 17.9; K 512, N 8192, 65 tokens in 1 / 2 9.9 /
-    // 12.0). INT4's costlier expansion keeps larger tiles
-    const int tiles = cdiv(p.M, 64) * n_tiles;
-    if (fmt == 1) {
-      bm = 32;
-      ksplit = std::min({4, kCusPerXcd / cdiv(cdiv(p.M, 32) * n_tiles, kXcds), p.K / 64 / 6});
-    } else if (p.M <= 128) {
-      ksplit = std::min(cdiv(256, tiles), std::max(1, (p.K / 64) / 8));
-    } else {
-      bm = 128;
-      ksplit = 4;
-    }
-    ksplit = std::max(1, std::min(ksplit, p.K / 64));
-  } else if (cdiv(p.M, 128) * n_tiles < 256) {
-    // Fewer than 256 128-token tiles: two K groups of wavefronts per
-    // workgroup, one workgroup per CU, in the largest tiles that put at least
-    // 130 workgroups on the 256 CUs, with K in up to 4 slices of at least 28
-    // stages; else 32-token tiles with slices of at least 16. Measured on
-    // MI355X (MXFP4): K 2880, N 5760 at 203 / 512 / 1024 tokens 19.3 / 29.5 /
-    // 47.5 us (32-, 64-, 128-token tiles; the others 26 / 37 / 57), K 14336,
-    // N 4096 at 203 / 512 42.1 / 69.5 (64-, 128-token tiles, 4 slices)
-    const int nu = p.K / 64;
-    bool found = false;
-    for (int b : {128, 64, 32}) {
-      const int t = cdiv(p.M, b) * n_tiles;
-      const int k = std::max(1, std::min({256 / std::max(t, 1), 4, nu / 28}));
-      if (t <= 256 && t * k >= 130) {
-        bm = b;
-        ksplit = k;
-        found = true;
-        break;
-      }
-    }
-    if (!found) {
-      bm = 32;
-      ksplit = std::max(1, std::min({256 / std::max(1, cdiv(p.M, 32) * n_tiles), 4, nu / 16}));
-    }
-  } else {
-    bm = 128;
-  }
+  const W4Plan plan = w4_choose(p, fmt, n_tiles);
+  const int bm = plan.bm, ksplit = plan.ksplit;
   const int m_tiles0 = p.group_offs ? cdiv(p.M, bm) + std::min(p.slots, p.M) : cdiv(p.M, bm);
   if ((int64_t)m_tiles0 * n_tiles > (1 << 30)) return false;
-  const char* ks_env = getenv("QMOE_W4_KSPLIT");  // tuning knob
-  if (ks_env && atoi(ks_env) > 0) ksplit = std::max(1, std::min(atoi(ks_env), p.K / 64));
   *bm_out = bm;
   *ksplit_out = ksplit;
   *ws_bytes = ksplit > 1 ? (int64_t)ksplit * p.M * p.N * 4 : 0;
@@ -983,18 +995,15 @@ int qmoe_w4_launch(GemmParams p, int fmt, void* workspace, int64_t ws_bytes, hip
     if (!workspace || ws_bytes < need) return QMOE_ERR_WORKSPACE;
     p.partial = static_cast<float*>(workspace);
   }
-  const int n_tiles = cdiv(p.act != QA_NONE ? p.N / 2 : p.N, p.act != QA_NONE ? kW4BN / 2 : kW4BN);
-  if (w4_ring(p, fmt, n_tiles)) {
-    if (fmt == 1) w4_ring_groups(p) == 2 ? w4_launch_ring<32, 2, 1>(p, st) : w4_launch_ring<32, 1, 1>(p, st);
-    else if (bm == 128) w4_launch_ring<128, 1, 2>(p, st);
-    else w4_launch_ring<64, 1, 2>(p, st);
+  const W4Plan plan =
+      w4_choose(p, fmt, cdiv(p.act != QA_NONE ? p.N / 2 : p.N, p.act != QA_NONE ? kW4BN / 2 : kW4BN));
+  if (plan.ring) {
+    if (fmt == 2) w4_launch_ring<64, 1, 2>(p, st);
+    else plan.kgroups == 2 ? w4_launch_ring<32, 2, 1>(p, st) : w4_launch_ring<32, 1, 1>(p, st);
   } else if (bm == 128) {
-    // two K groups of wavefronts per workgroup where one workgroup per CU is all there is
-    if (p.group_offs || cdiv(p.M, 128) * n_tiles * ksplit > 256) w4_launch_fmt<128, 1>(p, fmt, st);
-    else w4_launch_fmt<128, 2>(p, fmt, st);
+    plan.kgroups == 2 ? w4_launch_fmt<128, 2>(p, fmt, st) : w4_launch_fmt<128, 1>(p, fmt, st);
   } else if (bm == 64) {
-    if (p.group_offs) w4_launch_fmt<64, 1>(p, fmt, st);
-    else w4_launch_fmt<64, 2>(p, fmt, st);
+    plan.kgroups == 2 ? w4_launch_fmt<64, 2>(p, fmt, st) : w4_launch_fmt<64, 1>(p, fmt, st);
   } else {
     w4_launch_fmt<32, 2>(p, fmt, st);
   }
