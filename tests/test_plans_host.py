@@ -69,3 +69,17 @@ def test_forced_4bit_tile_height(monkeypatch, bm, kind, M):
     assert _plan(kind, M, 5760, 2880) == ("tiled_4b", bm, 1)
     monkeypatch.setenv("QMOE_W4_KSPLIT", "3")
     assert _plan(kind, M, 5760, 2880) == ("tiled_4b", bm, 3)
+
+
+@pytest.mark.parametrize("kind,E,M,N,K,act,tile", [
+    # weight tiles on one workgroup per CU, or one round of two per CU, in 64-token tiles
+    ("W4A16_MX", 4, 512, 5760, 2880, "silu", 64),
+    ("W4A16_MX", 8, 1024, 2880, 2880, None, 64),
+    ("W4A16_NV", 8, 1024, 5760, 2880, "silu", 64),
+    ("W4A16_MX", 16, 1024, 2880, 2880, None, 128),  # 288 64-token tiles, 192 of 128
+    ("W4A16_I4", 128, 128 * 64, 5760, 2880, "silu", 128),
+    ("W4A16_MX", 128, 128 * 40, 5760, 2880, "silu", 64),
+])
+def test_grouped_4bit_tile_heights(monkeypatch, kind, E, M, N, K, act, tile):
+    monkeypatch.setenv("QMOE_SKINNY_MAX_ROWS", "0")
+    assert _plan(kind, M, N, K, activation=act, experts=E) == ("tiled_4b", tile, 1)

@@ -929,13 +929,29 @@ W4Plan w4_plan_dense(const GemmParams& p, int fmt, int n_tiles, int force_bm, in
   return best;
 }
 
-// Routed experts, measured on MI355X (GPT-OSS MoE, 128 experts, MXFP4): 64
-// rows per routed expert 797 us in 64-token tiles (half of the experts need a
-// second one) and 696 in 128-token tiles, 32 rows 518 and 532.
-W4Plan w4_plan_grouped(const GemmParams& p, int force_bm, int force_ks) {
+// m-tiles of `bm` rows that the groups are expected to need
+int w4_group_tiles(const GemmParams& p, int bm) {
+  const int groups = std::max(1, std::min(p.slots, p.M));
+  return std::max(groups, p.M / bm + groups / 2);
+}
+
+// Routed experts. Tiles that about fill one workgroup per CU run two K groups
+// in each; beyond 40 rows per expert 128-token tiles, unless one round of
+// 64-token tiles (two workgroups per CU) holds them all. Measured on MI355X
+// (one group, 64 / 128 tokens; two groups, 64 / 128): MXFP4, 4 experts, K
+// 2880, N 5760, 16 rows each 27.6 / 29.7; 21.8 / 23.9 us, 128 rows 39.8 / 63.4;
+// 31.9 / 55.0; 8 experts, 128 rows 57.2 / 86.0; 64.9 / 105.7; 16 experts, N
+// 2880, 64 rows 50.2 / 46.6; 58.0 / 38.9; GPT-OSS MoE layer (128 experts), 32 /
+// 64 rows 518 / 797 in 64-token tiles, 532 / 696 in 128-token tiles.
+W4Plan w4_plan_grouped(const GemmParams& p, int n_tiles, int force_bm, int force_ks) {
+  constexpr int kFill = 272;  // the estimate, a little over 256
+  auto count = [&](int bm) { return (int64_t)w4_group_tiles(p, bm) * n_tiles; };
+  const int rows = p.M / std::max(1, std::min(p.slots, p.M));
   W4Plan r;
   if (force_bm) r.bm = std::max(force_bm, 64);
-  else r.bm = p.M / std::max(1, std::min(p.slots, p.M)) > 40 ? 128 : 64;
+  else if (count(64) <= kFill || rows <= 40) r.bm = 64;
+  else r.bm = count(128) <= kFill || count(64) > 512 ? 128 : 64;
+  r.kgroups = count(r.bm) <= kFill ? 2 : 1;
   r.ksplit = std::max(force_ks, 1);
   return r;
 }
@@ -948,7 +964,7 @@ W4Plan w4_choose(const GemmParams& p, int fmt, int n_tiles) {
   const int bm = env && (atoi(env) == 128 || atoi(env) == 64 || atoi(env) == 32) ? atoi(env) : 0;
   const char* ks_env = getenv("QMOE_W4_KSPLIT");
   const int ks = ks_env && atoi(ks_env) > 0 ? std::min(atoi(ks_env), p.K / 64) : 0;
-  return p.group_offs ? w4_plan_grouped(p, bm, ks) : w4_plan_dense(p, fmt, n_tiles, bm, ks);
+  return p.group_offs ? w4_plan_grouped(p, n_tiles, bm, ks) : w4_plan_dense(p, fmt, n_tiles, bm, ks);
 }
 
 }  // namespace
