@@ -83,3 +83,41 @@ def test_forced_4bit_tile_height(monkeypatch, bm, kind, M):
 def test_grouped_4bit_tile_heights(monkeypatch, kind, E, M, N, K, act, tile):
     monkeypatch.setenv("QMOE_SKINNY_MAX_ROWS", "0")
     assert _plan(kind, M, N, K, activation=act, experts=E) == ("tiled_4b", tile, 1)
+
+
+@pytest.mark.parametrize("kind,E,M,N,K,act,path", [
+    ("W4A16_MX", 8, 8, 2880, 2880, None, "stream"),  # 96 weight tiles
+    ("W4A16_MX", 8, 64, 5760, 2880, "silu", "stream"),
+    ("W4A16_MX", 32, 127, 2880, 2880, None, "stream"),  # 384, 3 rows each
+    ("W4A16_MX", 32, 128, 2880, 2880, None, "tiled_4b"),
+    ("W4A16_MX", 32, 32, 5760, 2880, "silu", "stream"),
+    ("W4A16_MX", 128, 127, 5760, 2880, "silu", "stream"),
+    ("W4A16_MX", 128, 128, 5760, 2880, "silu", "tiled_4b"),
+    ("W4A16_MX", 128, 128, 2880, 2880, None, "tiled_4b"),
+    ("W4A16_NV", 16, 128, 5760, 2880, "silu", "stream"),
+    ("W4A16_NV", 32, 160, 5760, 2880, "silu", "stream"),
+    ("W4A16_NV", 32, 192, 5760, 2880, "silu", "tiled_4b"),
+    ("W4A16_NV", 128, 1024, 1536, 2048, "silu", "stream"),
+    ("W4A16_NV", 128, 128, 2880, 2880, None, "tiled_4b"),
+    ("W4A16_I4", 128, 1024, 5760, 2880, "silu", "stream"),
+    ("W4A16_MX", 8, 128, 2880, 2880, None, "tiled_4b"),  # beyond the streaming kernel's rows
+])
+def test_grouped_4bit_streaming_limit(kind, E, M, N, K, act, path):
+    assert _plan(kind, M, N, K, activation=act, experts=E)[0] == path
+
+
+def test_grouped_4bit_operands_that_the_tiles_decline():
+    """Rows of scales of an odd length: streaming, sized by the rows per expert."""
+    from qmoe import _capi
+
+    d = _capi.GemmDesc()
+    d.kind, d.a, d.w, d.y, d.w_scale = _capi.W4A16_MX, 1 << 24, 1 << 24, 1 << 24, 1 << 24
+    d.lda, d.ldw, d.ldy, d.w_gstride = 2880, 1440, 2880, 1440 * 2880
+    d.group_offs = d.active = d.num_active = 1 << 24
+    d.M = d.max_rows = d.slots = 128
+    d.N = d.K = 2880
+    path, tile, ks = (ctypes.c_int32() for _ in range(3))
+    for ldws, want in ((90, 2), (91, 0)):
+        d.ldws, d.ws_gstride = ldws, ldws * 2880
+        assert _capi.lib.qmoe_gemm_plan(ctypes.byref(d), ctypes.byref(path), ctypes.byref(tile), ctypes.byref(ks)) == 0
+        assert path.value == want

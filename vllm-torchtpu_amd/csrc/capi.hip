@@ -166,11 +166,48 @@ int skinny_rows(const qmoe_gemm_desc* d) {
   return std::max(1, std::min(std::min(d->max_rows, d->M), avg));
 }
 
+// the W4A16 tiled kernel's format code: 0 MXFP4, 1 NVFP4, 2 INT4
+int w4_fmt(const qmoe_gemm_desc* d) {
+  return d->kind == QMOE_W4A16_NV ? 1 : (d->kind == QMOE_W4A16_I4 ? 2 : 0);
+}
+
+bool use_w4(const qmoe_gemm_desc* d) {
+  // the generic kernel has no NVFP4 / INT4 form
+  if (d->kind == QMOE_W4A16_NV || d->kind == QMOE_W4A16_I4) return true;
+  return d->kind == QMOE_W4A16_MX && !getenv("QMOE_W4_OFF");  // tuning knob: generic kernel only
+}
+
+// Grouped MXFP4 / NVFP4 that the tiles take from the streaming kernel although
+// its row limit would hold: `pairs`, the weight tiles of every expert (512 are
+// one round of the tiles), have to fill the chip, and below about three rounds
+// a tile's expansion has to serve several rows. Where the tiles decline the
+// operands, streaming keeps them. Measured on MI355X (streaming / tiles, us):
+// MXFP4, K 2880: 1472-1536 pairs (64 experts, N 5760; 128, N 2880) 1 row per
+// expert 98 / 86 and 86 / 80, 2 rows 132 / 119 and 129 / 114; 736 pairs (32
+// experts, N 5760) 1 / 2 / 4 / 8 rows 40 / 50 / 70 / 86 and 37 / 61 / 70 / 74;
+// 384 pairs (32, N 2880) 4 / 8 rows 33 / 39 and 33 / 33; 184 pairs (8, N 5760)
+// 1 / 8 rows 16 / 23 and 22 / 22. NVFP4: 1472-1536 pairs 1 row 125 / 112 and
+// 112 / 105; 736-768 pairs (32, N 5760; 64, N 2880) 2 / 6 rows 72 / 86 and 104
+// / 91, 68 / 82 and 104 / 94; 768 pairs of K 2048 (128, N 1536) 6 / 8 rows 61 /
+// 71 and 66 / 72. INT4 keeps the limit (GPT-OSS MoE, 32 / 128 tokens 355 / 577
+// streaming, 407 / 597 tiles).
+bool grouped_e2m1_tiles(const qmoe_gemm_desc* d, const GemmParams& p) {
+  if (!d->group_offs || (d->kind != QMOE_W4A16_MX && d->kind != QMOE_W4A16_NV) || d->M < d->slots) return false;
+  const int n_tiles = d->act != QMOE_ACT_NONE ? cdiv(d->N / 2, 128) : cdiv(d->N, 256);
+  const int64_t pairs = (int64_t)d->slots * n_tiles;
+  const int rows = d->M / std::max(1, d->slots);
+  const bool nv = d->kind == QMOE_W4A16_NV;
+  if (pairs < 1400 && (nv ? pairs < 700 || d->K < 2560 || rows < 6 : pairs < 350 || rows < 4)) return false;
+  int bm = 0, ks = 1;
+  int64_t ws = 0;
+  return use_w4(d) && qmoe_w4_plan(p, w4_fmt(d), &bm, &ks, &ws);
+}
+
 // Dense problems take the skinny kernel up to 64 rows (32 for W8A8, whose
 // tiled kernel is faster from there on); grouped ones while the routed
 // experts average at most 8 rows (measured on MI355X: beyond that the tiled
 // kernel's weight reuse across rows wins).
-bool use_skinny(const qmoe_gemm_desc* d) {
+bool use_skinny(const qmoe_gemm_desc* d, const GemmParams& p) {
   const char* env = getenv("QMOE_SKINNY_MAX_ROWS");  // tuning knob
   int lim = d->group_offs ? kSkinnyMaxGroupRows : kSkinnyMaxRows;
   if (!d->group_offs && (d->kind == QMOE_W8A8_PC || d->kind == QMOE_W8A8_GMM)) lim = kSkinnyMaxRowsW8A8;
@@ -185,27 +222,9 @@ bool use_skinny(const qmoe_gemm_desc* d) {
   // dense e2m1 (MXFP4 / NVFP4): the tiled kernel's 32-token tiles with a K
   // split win from 33 rows (measured on MI355X, K 2880, N 5760)
   if (!d->group_offs && (d->kind == QMOE_W4A16_MX || d->kind == QMOE_W4A16_NV)) lim = kSkinnyMaxRowsW8A8;
-  // grouped e2m1: the tiles from as many routes as experts on (measured on
-  // MI355X, GPT-OSS MoE, 128 experts, top 4: MXFP4 16 tokens 201 us both ways,
-  // 32 / 64 / 128 / 256 tokens 346 / 447 / 514 / 590 -> 316 / 373 / 403 / 419
-  // us, NVFP4 32 / 128 tokens 399 / 612 -> 392 / 541; INT4 loses, 355 / 577 ->
-  // 407 / 597)
-  if (d->group_offs && (d->kind == QMOE_W4A16_MX || d->kind == QMOE_W4A16_NV) && d->M >= d->slots &&
-      (d->K % 64) == 0)
-    lim = 0;
+  if (grouped_e2m1_tiles(d, p)) lim = 0;
   if (env) lim = atoi(env);
   return skinny_rows(d) <= lim;
-}
-
-// the W4A16 tiled kernel's format code: 0 MXFP4, 1 NVFP4, 2 INT4
-int w4_fmt(const qmoe_gemm_desc* d) {
-  return d->kind == QMOE_W4A16_NV ? 1 : (d->kind == QMOE_W4A16_I4 ? 2 : 0);
-}
-
-bool use_w4(const qmoe_gemm_desc* d) {
-  // the generic kernel has no NVFP4 / INT4 form
-  if (d->kind == QMOE_W4A16_NV || d->kind == QMOE_W4A16_I4) return true;
-  return d->kind == QMOE_W4A16_MX && !getenv("QMOE_W4_OFF");  // tuning knob: generic kernel only
 }
 
 bool use_f8(const qmoe_gemm_desc* d) {
@@ -341,14 +360,14 @@ int qmoe_route_of(const qmoe_gemm_desc* d, GemmParams& p, QmoeRoute* r) {
       return QMOE_OK;
     }
   }
-  if (use_skinny(d) && qmoe_skinny_check(kind, p) == QMOE_OK) {
+  if (use_skinny(d, p) && qmoe_skinny_check(kind, p) == QMOE_OK) {
     r->path = kPathSkinny;
     r->tile_m = qmoe_skinny_tile_rows(skinny_rows(d));
     qmoe_skinny_plan(kind, d->M, d->N, d->K, d->act, skinny_slots(d), skinny_rows(d), 0, &r->ksplit,
                      &r->ws_bytes);
     return QMOE_OK;
   }
-  const bool skinny_first = use_skinny(d);
+  const bool skinny_first = use_skinny(d, p);
   p.active = nullptr;
   p.num_active = nullptr;
   if (!skinny_first) {
