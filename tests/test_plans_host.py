@@ -121,3 +121,27 @@ def test_grouped_4bit_operands_that_the_tiles_decline():
         d.ldws, d.ws_gstride = ldws, ldws * 2880
         assert _capi.lib.qmoe_gemm_plan(ctypes.byref(d), ctypes.byref(path), ctypes.byref(tile), ctypes.byref(ks)) == 0
         assert path.value == want
+
+
+@pytest.mark.parametrize("kind,E,rows,N,K,act,want", [
+    # fewer than 200 tiles of 128 tokens: the four-wavefront tiles
+    ("W8A8_GMM", 8, 64, 4096, 7168, "silu", ("tiled_1b", 64)),
+    ("W8A8_BLK", 8, 96, 4096, 14336, None, ("tiled_1b_n128", 64)),
+    ("W8A8_GMM", 4, 200, 4096, 7168, "silu", ("tiled_1b", 128)),
+    ("W8A8_GMM", 8, 64, 7168, 2048, None, ("tiled_8w", 128)),
+    # tile-scaled, few rows, no activation: their 128-row weight tiles
+    ("W8A8_BLK", 32, 8, 7168, 2048, None, ("tiled_1b_n128", 32)),
+    ("W8A8_BLK", 32, 48, 7168, 2048, None, ("tiled_1b_n128", 64)),
+    ("W8A8_BLK", 32, 64, 7168, 2048, None, ("tiled_8w", 128)),
+    ("W8A8_BLK", 256, 48, 7168, 2048, None, ("tiled_8w", 128)),
+    ("W8A8_GMM", 32, 8, 7168, 2048, None, ("tiled_8w", 128)),
+    # tile heights by the rounds of tiles
+    ("W8A8_GMM", 64, 96, 4096, 7168, "silu", ("tiled_8w", 128)),
+    ("W8A8_GMM", 64, 128, 4096, 7168, "silu", ("tiled_8w", 256)),
+    ("W8A8_GMM", 64, 200, 4096, 7168, "silu", ("tiled_8w", 256)),
+    ("W8A8_GMM", 64, 300, 4096, 7168, "silu", ("tiled_8w", 128)),
+    ("W8A8_GMM", 256, 64, 4096, 7168, "silu", ("tiled_8w", 128)),
+    ("W8A8_GMM", 8, 64, 4096, 7168 + 128, "silu", ("tiled_8w", 128)),  # K outside the other tiles' granule
+])
+def test_grouped_fp8_plans(kind, E, rows, N, K, act, want):
+    assert _plan(kind, E * rows, N, K, activation=act, experts=E, ws_bn=128 if kind == "W8A8_BLK" else 1)[:2] == want

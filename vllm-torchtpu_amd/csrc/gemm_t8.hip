@@ -460,6 +460,27 @@ int t8_n_tiles(const GemmParams& p) {
   return cdiv(p.act != QA_NONE ? p.N / 2 : p.N, p.act != QA_NONE ? kT8BN / 2 : kT8BN);
 }
 
+// Token-tile height of routed experts, 0 for gemm_f8.hip's tiles. An expert is
+// taken to hold the average rows and a sixteenth more. A round of 256-token
+// tiles over the 256 CUs takes about 1.68 times one of 128-token tiles
+// (measured, 128 / 256, us: DeepSeek-V3 routed experts, K 7168, N 4096, 64
+// experts, 96 / 128 / 200 / 300 rows each 390 / 450, 576 / 486, 738 / 578, 921
+// / 1193; 8 experts, K 2048, N 7168, 128 / 300 rows 55 / 33, 76 / 89). Below
+// 200 tiles of 128 tokens the smaller ones of gemm_f8.hip put more CUs to work
+// (8 experts, K 7168, N 4096, 64 / 96 rows 51 / 56 us there, 56 / 70 here; K
+// 14336, N 4096, 96 rows 118 / 155), and so do its 128-row weight tiles for
+// tile-scaled experts of few rows without an activation (K 2048, N 7168: 32
+// experts, 8 / 48 rows 88 / 104 there, 94 / 110 here; 64 experts, 48 rows 198
+// both; 256 experts, 32 rows 768 / 736). `tiles`: weight scales per 128 x 128.
+int t8_grouped_tile(const GemmParams& p, bool tiles) {
+  const int groups = std::max(1, std::min(p.slots, p.M)), rows = p.M / groups;
+  const int64_t n = (int64_t)groups * t8_n_tiles(p);
+  auto tiles_of = [&](int bm) { return n * cdiv(rows + rows / 16, bm); };
+  if ((p.K % 256) == 0 && (rows == 0 ? n : tiles_of(128)) < 200) return 0;
+  if ((p.K % 256) == 0 && tiles && p.act == QA_NONE && rows <= 48 && n < 1024) return 0;
+  return cdiv<int64_t>(tiles_of(256), 256) * 168 < cdiv<int64_t>(tiles_of(128), 256) * 100 ? 256 : 128;
+}
+
 }  // namespace
 
 // Token-tile height of the problem on this kernel (256 also where the last
@@ -477,13 +498,7 @@ int qmoe_t8_plan(const GemmParams& p, bool f8) {
   if (!f8 && (p.group_offs || p.act != QA_NONE)) return 0;
   const char* env = getenv("QMOE_T8_BM");  // tuning knob: 128, 256 or 0 (off)
   if (env) return atoi(env) == 128 || atoi(env) == 256 ? atoi(env) : 0;
-  if (p.group_offs) {
-    // measured on MI355X (DeepSeek-V3 routed experts, 256 experts, top 8,
-    // per-channel weights; gemm_f8.hip's tiles, 128-, 256-token tiles): 64
-    // tokens 1041 / 1029 / 1025 us, 256 tokens 1414 / 1343 / 1503, 2048
-    // 2659 / 2356 / 2558, 8192 (128 x 128 tiles) 5989 / 5591 / 5162
-    return p.M / std::max(1, std::min(p.slots, p.M)) > 192 ? 256 : 128;
-  }
+  if (p.group_offs) return t8_grouped_tile(p, f8 && !wpc);
   // Dense, if it has work for more than half of the CUs; else the smaller
   // tiles and K splits of the other kernels (K 4096, N 4096, 1024 tokens, 128
   // tiles: 50 us here, 41 there; K 2048, N 7168, 1000 tokens, 224 tiles: 32
