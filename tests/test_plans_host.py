@@ -145,3 +145,10 @@ def test_grouped_4bit_operands_that_the_tiles_decline():
 ])
 def test_grouped_fp8_plans(kind, E, rows, N, K, act, want):
     assert _plan(kind, E * rows, N, K, activation=act, experts=E, ws_bn=128 if kind == "W8A8_BLK" else 1)[:2] == want
+
+
+@pytest.mark.parametrize("N,path", [(1, "tiled_generic"), (64, "tiled_generic"), (128, "tiled_generic"),
+                                    (129, "tiled_8w"), (256, "tiled_8w"), (257, "tiled_generic"),
+                                    (320, "tiled_generic"), (385, "tiled_8w"), (576, "tiled_8w"), (640, "tiled_8w")])
+def test_bf16_width_that_256_row_tiles_pad(N, path):
+    assert _plan("W16A16", 40000, N, 2880)[0] == path

@@ -504,6 +504,10 @@ int qmoe_t8_plan(const GemmParams& p, bool f8) {
   // tiles: 50 us here, 41 there; K 2048, N 7168, 1000 tokens, 224 tiles: 32
   // and 42).
   const int n_tiles = t8_n_tiles(p), tall = t8_tall_tiles(p.M, n_tiles);
+  // bf16 of a width that 256-row tiles pad by a third or more over the generic
+  // tiles' 128 rows: up to 128 channels and 257 to 384 (K 2880, 40000 tokens, N
+  // 64 / 320: 76 / 135 us here, 58 / 121 there; N 640 184 here, 209 there)
+  if (!f8 && 3 * 2 * cdiv(p.N, 256) >= 4 * cdiv(p.N, 128)) return 0;
   const int64_t tiles = (int64_t)(tall + cdiv(std::max(p.M - (int64_t)tall * 256, (int64_t)0), (int64_t)128)) * n_tiles;
   return tiles >= 140 ? (tall ? 256 : 128) : 0;
 }
