@@ -152,3 +152,13 @@ def test_grouped_fp8_plans(kind, E, rows, N, K, act, want):
                                     (320, "tiled_generic"), (385, "tiled_8w"), (576, "tiled_8w"), (640, "tiled_8w")])
 def test_bf16_width_that_256_row_tiles_pad(N, path):
     assert _plan("W16A16", 40000, N, 2880)[0] == path
+
+
+@pytest.mark.parametrize("M,N,K,want", [
+    (256, 24576, 1536, ("tiled_8w", 128)), (257, 24576, 1536, ("tiled_1b_n128", 64)),
+    (320, 24576, 7168, ("tiled_1b_n128", 64)), (321, 24576, 7168, ("tiled_8w", 256)),
+    (300, 18432, 7168, ("tiled_8w", 128)),  # 216 tiles: one round
+    (300, 24576, 7168 + 128, ("tiled_8w", 256)),  # K outside the other tiles' granule
+])
+def test_block_fp8_of_257_to_320_tokens(M, N, K, want):
+    assert _plan("W8A8_BLK", M, N, K, ws_bn=128)[:2] == want

@@ -508,6 +508,11 @@ int qmoe_t8_plan(const GemmParams& p, bool f8) {
   // tiles' 128 rows: up to 128 channels and 257 to 384 (K 2880, 40000 tokens, N
   // 64 / 320: 76 / 135 us here, 58 / 121 there; N 640 184 here, 209 there)
   if (!f8 && 3 * 2 * cdiv(p.N, 256) >= 4 * cdiv(p.N, 128)) return 0;
+  // block-scaled, 257 to 320 tokens over more than one round of 128-token tiles:
+  // five 64-token tiles pad less than three of 128 or two of 256 (300 tokens, K
+  // 1536 / 7168, N 24576: 36 / 114 us here, 30 / 97 there; one round, K 7168, N
+  // 18432: 69 here, 74 there)
+  if (f8 && p.act == QA_NONE && (p.K % 256) == 0 && p.M > 256 && p.M <= 320 && 3 * (int64_t)n_tiles > 256) return 0;
   const int64_t tiles = (int64_t)(tall + cdiv(std::max(p.M - (int64_t)tall * 256, (int64_t)0), (int64_t)128)) * n_tiles;
   return tiles >= 140 ? (tall ? 256 : 128) : 0;
 }
