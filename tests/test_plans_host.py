@@ -76,6 +76,7 @@ def test_forced_4bit_tile_height(monkeypatch, bm, kind, M):
     ("W4A16_MX", 4, 512, 5760, 2880, "silu", 64),
     ("W4A16_MX", 8, 1024, 2880, 2880, None, 64),
     ("W4A16_NV", 8, 1024, 5760, 2880, "silu", 64),
+    ("W4A16_MX", 4, 1200, 5760, 2880, "silu", 64),  # 276 128-token tiles of equal experts
     ("W4A16_MX", 16, 1024, 2880, 2880, None, 128),  # 288 64-token tiles, 192 of 128
     ("W4A16_I4", 128, 128 * 64, 5760, 2880, "silu", 128),
     ("W4A16_MX", 128, 128 * 40, 5760, 2880, "silu", 64),

@@ -929,10 +929,11 @@ W4Plan w4_plan_dense(const GemmParams& p, int fmt, int n_tiles, int force_bm, in
   return best;
 }
 
-// m-tiles of `bm` rows that the groups are expected to need
+// m-tiles of `bm` rows that the groups are expected to need: those of equal
+// groups, or of groups whose last tiles are half filled on average
 int w4_group_tiles(const GemmParams& p, int bm) {
   const int groups = std::max(1, std::min(p.slots, p.M));
-  return std::max(groups, p.M / bm + groups / 2);
+  return std::max(groups * cdiv(p.M / groups, bm), p.M / bm + groups / 2);
 }
 
 // Routed experts. Tiles that about fill one workgroup per CU run two K groups
