@@ -90,7 +90,9 @@ def test_grouped(monkeypatch, bm, recipe, N, K, act):
                         a_rows=rows, activation=act, row_weight=rw, y_rows=perm, out=out)
 
     monkeypatch.setenv("QMOE_SKINNY_MAX_ROWS", "0")
-    got = run(bm)
+    with ops.record_plans() as plans:
+        got = run(bm)
+    assert tuple(plans[0][4:]) == ("tiled_8w", int(bm), 1)
     if K % 256 == 0:
         base = run("0")
         if tiles:
@@ -136,37 +138,62 @@ def test_bf16(monkeypatch, bm, M, N, K):
     _check(got, x.double() @ w.double().t() + bias.double(), x.double().abs() @ w.double().abs().t() + bias.double().abs())
 
 
+def _tall_tiles(M, N):
+    """256-token tiles ahead of a dense problem's 128-token ones: the fewest
+    weighted rounds over 256 CUs (256-token tiles 168, 128-token ones 100, a
+    second launch 10), tall rounds whole but for the last or the last two."""
+    nt = -(-N // 256)
+    m256 = -(-M // 256)
+    rounds = -(-m256 * nt // 256)
+    tall = [0, m256] + [r * 256 // nt for r in range(rounds - 1, 0, -1) if r >= rounds - 2]
+
+    def cost(t):
+        rest = max(M - 256 * t, 0)
+        return -(-t * nt // 256) * 168 + -(-(-(-rest // 128) * nt) // 256) * 100 + (10 if t and rest else 0)
+
+    return min(tall, key=cost)
+
+
 @pytest.mark.parametrize("kind", ["fp8", "bf16"])
-@pytest.mark.parametrize("M,N", [(1024, 18432), (2047, 18432), (1500, 14300), (769, 18300)])
-def test_dense_rounds_of_two_heights(monkeypatch, kind, M, N):
+@pytest.mark.parametrize("M,N,K,two", [(1024, 18432, 256, True), (2047, 18432, 1152, True), (1500, 14300, 256, True),
+                                       (769, 18300, 256, False)])
+def test_dense_rounds_of_two_heights(monkeypatch, kind, M, N, K, two):
     """Problems whose last, partly filled round of 256-token tiles runs as
     128-token tiles (the last of the four: all in one height): the same sums
-    in the same order as 128-token tiles throughout."""
+    in the same order as 128-token tiles throughout, also from padded and
+    gathered activation rows."""
     from qmoe import _capi, ops
 
     g = _gen(M + N)
-    K = 256
     rw = torch.rand(M, device="cuda", generator=g).to(torch.bfloat16)
     perm = torch.randperm(M, generator=torch.Generator().manual_seed(3)).to(dtype=torch.int32, device="cuda")
+    rows = torch.randint(0, M, (M,), generator=g, dtype=torch.int32, device="cuda")
     if kind == "fp8":
         N = (N + 127) // 128 * 128
-        x, w = _codes((M, K), g), _codes((N, K), g)
-        xs, ws = _scales((M, K // 128), g), _scales((N // 128, K // 128), g)
+        x, w = _codes((M, K + 16), g)[:, :K], _codes((N, K), g)
+        xs, ws = _scales((M, K // 128 + 3), g)[:, :K // 128], _scales((N // 128, K // 128), g)
         call = lambda **kw: ops.gemm(_capi.W8A8_BLK, x.view(torch.uint8), w.view(torch.uint8), a_scale=xs,  # noqa: E731
                                      w_scale=ws, ws_bn=128, **kw)
         xd = x.double() * xs.double().repeat_interleave(128, 1)
         wd = w.double() * ws.double().repeat_interleave(128, 0).repeat_interleave(128, 1)
     else:
-        x = torch.randn((M, K), device="cuda", generator=g).to(torch.bfloat16)
+        x = torch.randn((M, K + 8), device="cuda", generator=g).to(torch.bfloat16)[:, :K]
         w = torch.randn((N, K), device="cuda", generator=g).to(torch.bfloat16)
         call = lambda **kw: ops.gemm(_capi.W16A16, x, w, **kw)  # noqa: E731
         xd, wd = x.double(), w.double()
-    for kw in ({}, dict(row_weight=rw, y_rows=perm)):
+    assert (0 < 256 * _tall_tiles(M, N) < M) == two
+    ref, mag = xd @ wd.t(), xd.abs() @ wd.abs().t()
+    for kw in ({}, dict(row_weight=rw, y_rows=perm), dict(a_rows=rows)):
         monkeypatch.delenv("QMOE_T8_BM", raising=False)
         with ops.record_plans() as plans:
             got = call(**kw)
-        assert plans[0][4] == "tiled_8w"
+        assert tuple(plans[0][4:6]) == ("tiled_8w", 256 if _tall_tiles(M, N) else 128)
         monkeypatch.setenv("QMOE_T8_BM", "128")
         assert torch.equal(got, call(**kw))
-        if not kw:
-            _check(got, xd @ wd.t(), xd.abs() @ wd.abs().t())
+        if "y_rows" in kw:
+            wt = rw.double()[:, None]
+            _check(got[perm.long()], ref * wt, mag * wt)
+        elif kw:
+            _check(got, ref[rows.long()], mag[rows.long()])
+        else:
+            _check(got, ref, mag)

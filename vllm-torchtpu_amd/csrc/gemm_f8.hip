@@ -1193,7 +1193,9 @@ static int f8_pick_bm_any(const GemmParams& p) {
   const int n_tiles = cdiv(nout, p.act != QA_NONE ? 128 : 256);
   if (p.group_offs) {
     // measured on MI355X (DeepSeek-V3 MoE, 256 experts): 64-token tiles
-    // also below 48 rows per routed expert (32-token tiles lose ~5%)
+    // also below 48 rows per routed expert (32-token tiles lose ~5%). FP8
+    // experts that fill the chip run gemm_t8.hip's tiles; these take int8
+    // codes and few experts
     const int avg = std::max(1, p.M / std::max(1, std::min(p.slots, p.M)));
     if (avg > 192) return 256;
     if (avg > 96) return 128;
@@ -1226,7 +1228,9 @@ bool qmoe_f8_plan(const GemmParams& p, bool blk, int* bm_out, int* ksplit_out, i
   const bool env_bm = getenv("QMOE_F8_BM") != nullptr;
   // dense block-scaled problems with at least 64 weight-row tiles (16384
   // output channels: DeepSeek-V3's wide projections) take the tile height
-  // and K split measured best on MI355X (K 7168, N 18432 / 24576)
+  // and K split measured best on MI355X (K 7168, N 18432 / 24576; e4m3 codes.
+  // From 140 tiles of 128 tokens on, but for 257 to 320 tokens, e4m3 problems
+  // run gemm_t8.hip's tiles and these rules are left to e5m2 and int8 codes)
   const int nout = p.act != QA_NONE ? p.N / 2 : p.N;
   const bool blk_wide = blk && !p.group_offs && cdiv(nout, p.act != QA_NONE ? 128 : 256) >= 64;
   if (blk && !env_bm) {
@@ -1303,7 +1307,10 @@ bool qmoe_f8_plan(const GemmParams& p, bool blk, int* bm_out, int* ksplit_out, i
   // Grouped 128 x 128-tile problems without an activation (the MoE down
   // projection) in 32- or 64-token tiles: 128-row weight tiles, measured on
   // MI355X (DeepSeek-V3 layer, native tiles) T = 256 / 512 1373.6 / 1566.8
-  // -> 1319.1 / 1517.9 us; 128-token tiles (T = 4096) lose with them
+  // -> 1319.1 / 1517.9 us; 128-token tiles (T = 4096) lose with them. e4m3
+  // codes come here with up to 48 rows per expert and under 1024 weight tiles
+  // over all experts, or under 200 tiles (32 experts, K 2048, N 7168, 8 rows 88
+  // us, 94 in gemm_t8.hip's tiles)
   if (blk && p.group_offs && !f8_wpc(p) && p.act == QA_NONE && !env_bm && bm <= 64) bn = 128;
   const char* env_bn = getenv("QMOE_F8_BN");  // tuning knob: 128 or 256
   if (env_bn && (p.act == QA_NONE || (blk && bm == 128))) bn = atoi(env_bn) == 128 ? 128 : 256;
