@@ -13,11 +13,10 @@
 //  * Output tile BM tokens x 256 weight rows; wavefront (wn, wm), wn < 4,
 //    wm < 2, owns 64 weight rows (two 32-row blocks) and the 32-token blocks
 //    wm, wm + 2, ..., so that a tile with few tokens loads both halves alike.
-//    Measured (DeepSeek-V3 gate_up, K 7168, N 18432, 2048 / 8192 tokens): 389 /
-//    1497 -> 354 / 1246 us; routed experts (256, top 8), 2048 tokens: 2659 ->
-//    2356 us; bf16 K 4096, N 6144, 1024 tokens 84 -> 62 us. What is left is
-//    the copies: 64 KB per stage of 2048 MFMA cycles, where the L2 delivers
-//    about 29 bytes per cycle and CU.
+//    Measured against the four-wavefront and generic tiles (block FP8 K 7168, N
+//    18432, 2048 / 8192 tokens, quantization included: 396 / 1516 -> 339 / 1223
+//    us; DeepSeek-V3 routed experts, 2048 tokens 2530 -> 2252 us; bf16 K 4096, N
+//    6144, 1024 tokens 78.6 -> 59.3 us).
 //  * Stages of 128 bytes of every row (128 e4m3 / 64 bf16 values), copied
 //    straight into a ring of LDS stages (two of 64 KB for 256 tokens, three of
 //    48 KB for 128); one barrier per stage.
@@ -38,8 +37,8 @@ constexpr int kT8BN = 256;
 
 __device__ __forceinline__ int t8_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
 
-// Wait until at most n vector-memory operations are outstanding, n < 12 known
-// at run time (wave-uniform)
+// Wait until at most n vector-memory operations are outstanding; n, known at
+// run time (wave-uniform), is one stage's copies, 4 to 7 (else: all)
 __device__ __forceinline__ void t8_wait(int n) {
   switch (n) {
     case 4: wait_copies_upto<4>(); break;
@@ -334,8 +333,6 @@ __global__ __launch_bounds__(kT8Threads, 2) void t8_gemm_kernel(const GemmParams
     s_bs[tid] = e_bs;
     s_ws[tid] = e_ws;
   }
-  const bool vec_ok = ((p.ldy & 7) == 0) && ((reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
-  const bool has_bias = p.bias != nullptr;
 #pragma unroll
   for (int j = 0; j < MJ; ++j) {
     if (j * 64 >= rows_u) break;
@@ -349,48 +346,7 @@ __global__ __launch_bounds__(kT8Threads, 2) void t8_gemm_kernel(const GemmParams
             make_float4(acc[i][j][q * 4], acc[i][j][q * 4 + 1], acc[i][j][q * 4 + 2], acc[i][j][q * 4 + 3]);
       }
     __syncthreads();
-    auto quad = [&](int t, int n) {
-      return *reinterpret_cast<const float4*>(reg + t * BN + (n ^ (4 * (t & 15))));
-    };
-    for (int e = tid; e < 64 * (BNO / 8); e += kT8Threads) {
-      const int t = e / (BNO / 8), c = (e % (BNO / 8)) * 8;  // token of the 64, first tile channel
-      const int tr = j * 64 + t;
-      if (tr >= rows || n0 + c >= nlim) continue;
-      const float4 g0 = quad(t, c), g1 = quad(t, c + 4);
-      const float vg[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-      float vu[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (ACT) {
-        const float4 h0 = quad(t, BN / 2 + c), h1 = quad(t, BN / 2 + c + 4);
-        vu[0] = h0.x; vu[1] = h0.y; vu[2] = h0.z; vu[3] = h0.w;
-        vu[4] = h1.x; vu[5] = h1.y; vu[6] = h1.z; vu[7] = h1.w;
-      }
-      const float rwt = s_rw[tr];
-      uint32_t packed[4];
-#pragma unroll
-      for (int k = 0; k < 8; k += 2) {
-        float o2[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          float v = vg[k + h];
-          if constexpr (F8 && WPC) v = v * s_ws[c + k + h];
-          if (has_bias) v += s_bs[c + k + h];
-          if (ACT) {
-            float u = vu[k + h];
-            if constexpr (F8 && WPC) u = u * s_ws[BN / 2 + c + k + h];
-            if (has_bias) u += s_bs[BN / 2 + c + k + h];
-            v = qmoe_act(p.act, v, u, p.act_p0, p.act_p1);
-          }
-          o2[h] = v * rwt;
-        }
-        packed[k / 2] = (uint32_t)f32_to_bf16(o2[0]) | ((uint32_t)f32_to_bf16(o2[1]) << 16);
-      }
-      uint16_t* dst = p.y + (int64_t)s_yr[tr] * p.ldy + n0 + c;
-      if (vec_ok && n0 + c + 8 <= nlim) {
-        *reinterpret_cast<uint4*>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-      } else {
-        for (int k = 0; k < 8 && n0 + c + k < nlim; ++k) dst[k] = (uint16_t)(packed[k / 2] >> ((k & 1) * 16));
-      }
-    }
+    tile_finish_rows<64, kT8Threads, BN, ACT, F8 && WPC>(p, reg, tid, j * 64, rows, n0, nlim, s_rw, s_bs, s_ws, s_yr);
   }
 }
 

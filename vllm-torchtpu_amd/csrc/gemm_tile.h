@@ -411,6 +411,66 @@ __device__ __forceinline__ void tile_epilogue(const GemmParams& p, const AccT (&
 // partials, the per-channel weight scale is not: the grouped-matmul recipe).
 enum { kScAll = 0, kScNone = 1, kScWeight = 2 };
 
+// A tile's f32 sums in LDS, [tokens][BN tile rows], token-major: the quad at
+// row n of token t, whose rows lie at n ^ 4 (t % 16) against bank conflicts.
+template <int BN>
+__device__ __forceinline__ float4 tile_quad(const float* sums, int t, int n) {
+  return *reinterpret_cast<const float4*>(sums + t * BN + (n ^ (4 * (t & 15))));
+}
+
+// Finish of a tile's tokens t0 .. t0 + T - 1 from their sums in LDS (tile_quad's
+// layout; with ACT gate rows, then up rows) by NT threads, 8 output channels of
+// a token each: weight scale per row (WSC), bias, fused activation, routing
+// weight, bf16, the output row of the token. s_*: per-token routing weights and
+// output rows, per-row bias and weight scales.
+template <int T, int NT, int BN, bool ACT, bool WSC>
+__device__ __forceinline__ void tile_finish_rows(const GemmParams& p, const float* sums, int tid, int t0, int rows,
+                                                 int n0, int nlim, const float* s_rw, const float* s_bs,
+                                                 const float* s_ws, const int* s_yr) {
+  constexpr int BNO = ACT ? BN / 2 : BN;
+  const bool vec_ok = ((p.ldy & 7) == 0) && ((reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
+  const bool has_bias = p.bias != nullptr;
+  for (int e = tid; e < T * (BNO / 8); e += NT) {
+    const int t = e / (BNO / 8), c = (e % (BNO / 8)) * 8;  // token of the T, first tile channel
+    const int tr = t0 + t;
+    if (tr >= rows || n0 + c >= nlim) continue;
+    const float4 g0 = tile_quad<BN>(sums, t, c), g1 = tile_quad<BN>(sums, t, c + 4);
+    const float vg[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+    float vu[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (ACT) {
+      const float4 h0 = tile_quad<BN>(sums, t, BN / 2 + c), h1 = tile_quad<BN>(sums, t, BN / 2 + c + 4);
+      vu[0] = h0.x; vu[1] = h0.y; vu[2] = h0.z; vu[3] = h0.w;
+      vu[4] = h1.x; vu[5] = h1.y; vu[6] = h1.z; vu[7] = h1.w;
+    }
+    const float rwt = s_rw[tr];
+    uint32_t packed[4];
+#pragma unroll
+    for (int k = 0; k < 8; k += 2) {
+      float o2[2];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        float v = vg[k + h];
+        if constexpr (WSC) v = v * s_ws[c + k + h];
+        if (has_bias) v += s_bs[c + k + h];
+        if (ACT) {
+          float u = vu[k + h];
+          if constexpr (WSC) u = u * s_ws[BN / 2 + c + k + h];
+          if (has_bias) u += s_bs[BN / 2 + c + k + h];
+          v = qmoe_act(p.act, v, u, p.act_p0, p.act_p1);
+        }
+        o2[h] = v * rwt;
+      }
+      packed[k / 2] = (uint32_t)f32_to_bf16(o2[0]) | ((uint32_t)f32_to_bf16(o2[1]) << 16);
+    }
+    uint16_t* dst = p.y + (int64_t)s_yr[tr] * p.ldy + n0 + c;
+    if (vec_ok && n0 + c + 8 <= nlim) {
+      *reinterpret_cast<uint4*>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
+    } else {
+      for (int k = 0; k < 8 && n0 + c + k < nlim; ++k) dst[k] = (uint16_t)(packed[k / 2] >> ((k & 1) * 16));
+    }
+  }
+}
+
 template <bool INT, bool ACT, int SC>
 __global__ __launch_bounds__(kThreads) void tile_splitk_finish_kernel(const GemmParams p) {
   constexpr bool SCALED = SC == kScNone;

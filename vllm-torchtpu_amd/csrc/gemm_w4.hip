@@ -19,17 +19,18 @@
 //    only fill one workgroup per CU: one wavefront's instructions issue in
 //    order, and it takes a second one to put the expansion of one beside the
 //    MFMAs of the other;
-//  * what bounds it: from ~1000 tokens the matrix cores and the copies into
-//    LDS beside them (K 2880, N 5760, 8192 tokens: 258 us, 1.05 PFLOP/s; MFMAs
-//    and LDS reads alone 172 us); a routed expert's few rows, the weight
-//    stream (GPT-OSS MoE, 512 / 2048 tokens 794 / 1162 -> 457 / 700 us);
+//  * what bounds it: from ~1000 tokens the expansion, the MFMAs and the copies
+//    into LDS, which overlap in part only (K 2880, N 5760, 4096 / 8192 tokens
+//    133 / 258 us, 1.05 PFLOP/s; MFMAs busy 41 % of the SIMDs' cycles); a
+//    routed expert's few rows, the weight stream as well (GPT-OSS MoE, 512 /
+//    2048 tokens 794 / 1112 us in 64-byte pieces -> 457 / 654 us; its gate_up
+//    fetches 1.36 GB for 1.13 GB of codes and scales);
 //  * a wavefront's codes are copied as whole 128-byte lines of its own rows
 //    (256 k, four stages) into its own LDS rows and from there into
 //    registers at the start of the line, which frees the buffer for the next
 //    line: 64 KB per CU stay in flight. 64-byte pieces of rows of 1440 bytes
-//    fetched 2.3 times the bytes (L2 misses 5.3 GB where the codes are 1.06
-//    GB) and were the limit. A wavefront owns every fourth row of the tile,
-//    whose lines start at the same place (see `ph`);
+//    touch a line more often than it stays in the L2. A wavefront owns every
+//    fourth row of the tile, whose lines start at the same place (see `ph`);
 //  * activations: stages of 64 k (128 bytes of each row) in a ring of three
 //    sets, copied two sets ahead, one barrier per set;
 //  * in a stage, lane l (row l % 32, half h = l / 32) feeds k in
@@ -416,8 +417,6 @@ __global__ __launch_bounds__(KG * kThreads, 2) void w4_gemm_kernel(const GemmPar
     s_yr[tid] = e_yr;
   }
   if (tid < BN) s_bs[tid] = e_bs;
-  const bool vec_ok = ((p.ldy & 7) == 0) && ((reinterpret_cast<uintptr_t>(p.y) & 15) == 0);
-  const bool has_bias = p.bias != nullptr;
 #pragma unroll
   for (int j = 0; j < MJ; ++j) {
     if (j * 32 >= rows_u) break;
@@ -436,9 +435,6 @@ __global__ __launch_bounds__(KG * kThreads, 2) void w4_gemm_kernel(const GemmPar
       }
       __syncthreads();
     }
-    auto quad = [&](int t, int n) {
-      return *reinterpret_cast<const float4*>(reg + t * BN + (n ^ (4 * (t & 15))));
-    };
     if (p.ksplit > 1) {
       // raw sums to the f32 workspace [ksplit][M][N]; the finishing kernel
       // adds the slices in order and runs the epilogue
@@ -448,7 +444,7 @@ __global__ __launch_bounds__(KG * kThreads, 2) void w4_gemm_kernel(const GemmPar
         const int tr = j * 32 + t;
         const int c = n0 + (ACT ? r % (BN / 2) : r);  // output channel of the quad
         if (tr >= rows || c >= nlim) continue;
-        const float4 v = quad(t, r);
+        const float4 v = tile_quad<BN>(reg, t, r);
         float* dst = plane + (int64_t)(row0 + tr) * p.N + (ACT && r >= BN / 2 ? p.N / 2 : 0) + c;
         if (c + 4 <= nlim && (p.N & 3) == 0 && (!ACT || (p.N & 7) == 0)) {
           *reinterpret_cast<float4*>(dst) = v;
@@ -459,43 +455,7 @@ __global__ __launch_bounds__(KG * kThreads, 2) void w4_gemm_kernel(const GemmPar
       }
       continue;
     }
-    for (int e = tid; e < 32 * (BNO / 8); e += NT) {
-      const int t = e / (BNO / 8), c = (e % (BNO / 8)) * 8;  // token of the block, first tile channel
-      const int tr = j * 32 + t;
-      if (tr >= rows || n0 + c >= nlim) continue;
-      const float4 g0 = quad(t, c), g1 = quad(t, c + 4);
-      const float vg[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
-      float vu[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-      if (ACT) {
-        const float4 h0 = quad(t, BN / 2 + c), h1 = quad(t, BN / 2 + c + 4);
-        vu[0] = h0.x; vu[1] = h0.y; vu[2] = h0.z; vu[3] = h0.w;
-        vu[4] = h1.x; vu[5] = h1.y; vu[6] = h1.z; vu[7] = h1.w;
-      }
-      const float rwt = s_rw[tr];
-      uint32_t packed[4];
-#pragma unroll
-      for (int k = 0; k < 8; k += 2) {
-        float o2[2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          float v = vg[k + h];
-          if (has_bias) v += s_bs[c + k + h];
-          if (ACT) {
-            float u = vu[k + h];
-            if (has_bias) u += s_bs[BN / 2 + c + k + h];
-            v = qmoe_act(p.act, v, u, p.act_p0, p.act_p1);
-          }
-          o2[h] = v * rwt;
-        }
-        packed[k / 2] = (uint32_t)f32_to_bf16(o2[0]) | ((uint32_t)f32_to_bf16(o2[1]) << 16);
-      }
-      uint16_t* dst = p.y + (int64_t)s_yr[tr] * p.ldy + n0 + c;
-      if (vec_ok && n0 + c + 8 <= nlim) {
-        *reinterpret_cast<uint4*>(dst) = make_uint4(packed[0], packed[1], packed[2], packed[3]);
-      } else {
-        for (int k = 0; k < 8 && n0 + c + k < nlim; ++k) dst[k] = (uint16_t)(packed[k / 2] >> ((k & 1) * 16));
-      }
-    }
+    tile_finish_rows<32, NT, BN, ACT, false>(p, reg, tid, j * 32, rows, n0, nlim, s_rw, s_bs, nullptr, s_yr);
   }
 }
 
@@ -518,9 +478,12 @@ struct W4Shape {
 // four stages ahead, with the operand reads and copies of a stage spread
 // over its MFMAs. It spends fewer instructions per stage than the line
 // pipeline above, and with one workgroup per CU that is what counts: NVFP4 K
-// 2880, N 5760 at 128 / 203 tokens 22.6 / 27.7 us against 26.0 / 32.0. The
-// expansion bounds it: two K groups of four wavefronts (KG 2, their sums added
-// through LDS) take 0.84 us per stage of each, one alone 0.50.
+// 2880, N 5760 at 128 / 203 tokens 22.6 / 27.7 us against 26.0 / 32.0. What
+// bounds it are the chains of a stage -- waits, barrier, operand reads, about
+// 180 vector instructions of expansion and few MFMAs (203 tokens: vector ALU
+// busy 23 % of the wave-cycles, MFMAs 7 % of the SIMDs'): two K groups of four
+// wavefronts (KG 2, their sums added through LDS) take 0.84 us per stage of
+// each, one alone 0.50.
 template <int BM, int KG, bool ACT, int FMT>
 __global__ __launch_bounds__(KG * kThreads) void w4_ring_kernel(const GemmParams p, int m_tiles, int n_tiles) {
   constexpr bool NV = FMT == 1, I4 = FMT == 2;
