@@ -49,6 +49,21 @@ __device__ __forceinline__ void t8_wait(int n) {
   }
 }
 
+// lds_copy16 (gemm_tile.h) of four offsets from one scalar base, to `lds` + 0,
+// 8, 16 and 24 KB: the move of the base that its wait states need, once for the
+// four (bf16 K 4096, N 6144, 1024 tokens 60.4 -> 59.5 us).
+__device__ __forceinline__ void t8_copy4(const uint8_t* base, const uint32_t (&off)[4], uint32_t lds) {
+  const uint8_t* b;
+  asm volatile(
+      "s_mov_b64 %0, %6\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %0\n\t"
+      "s_add_u32 m0, m0, 0x2000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %3, %0\n\t"
+      "s_add_u32 m0, m0, 0x2000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %4, %0\n\t"
+      "s_add_u32 m0, m0, 0x2000\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %5, %0"
+      : "=&s"(b)
+      : "s"(lds), "v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base)
+      : "m0", "scc", "memory");
+}
+
 // F8: block-scaled 1-byte floats; else bf16. WPC (F8): one weight scale per
 // weight row, applied in the epilogue, instead of one per 128 x 128 tile. WF:
 // weight format code of the MFMA, 0 e4m3, 1 e5m2 (activations are e4m3).
@@ -141,8 +156,8 @@ __global__ __launch_bounds__(kT8Threads, 2) void t8_gemm_kernel(const GemmParams
     const uint8_t* ws = reinterpret_cast<const uint8_t*>(
         (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(b >> 32)) << 32 |
         (uint32_t)__builtin_amdgcn_readfirstlane((int)b));
-#pragma unroll
-    for (int j = 0; j < WI; ++j) lds_copy16(ws, woff[j], d + j * 8192);
+    static_assert(WI == 4, "weight copies of a stage");
+    t8_copy4(ws, woff, d);
 #pragma unroll
     for (int j = 0; j < XI; ++j)
       if (j < nx) lds_copy16(xp[j] + (int64_t)s * 128, d + WB + j * 8192);
